@@ -328,7 +328,7 @@ int add_case(hc_context* ctx, int ni, int nj, const double* nodes, const hc_case
     return HC_OK;
 }
 
-template <class RF> void fill_rec(const hc_context* ctx, const CaseHost& c, int k, CaseRec<RF>& r)
+template <class RF> void fill_rec(const hc_context* ctx, const CaseHost& c, CaseRec<RF>& r)
 {
     r = CaseRec<RF>{};
     r.m.ni = c.ni;
@@ -341,14 +341,14 @@ template <class RF> void fill_rec(const hc_context* ctx, const CaseHost& c, int 
     r.m.ccx = ctx->ccx + c.geo_cell_off;
     r.m.ccy = ctx->ccy + c.geo_cell_off;
     if constexpr (sizeof(RF) == 8) {
-        r.m.fi = ctx->fi + NSLOT * c.geo_fi_off;
-        r.m.fj = ctx->fj + NSLOT * c.geo_fj_off;
+        r.m.fi = ctx->fi + ctx->nslot64() * c.geo_fi_off;
+        r.m.fj = ctx->fj + ctx->nslot64() * c.geo_fj_off;
     } else {
         r.m.fi = ctx->fi32 + NSLOT * c.geo_fi_off;
         r.m.fj = ctx->fj32 + NSLOT * c.geo_fj_off;
     }
-    r.m.fi64 = ctx->fi + NSLOT * c.geo_fi_off;
-    r.m.fj64 = ctx->fj + NSLOT * c.geo_fj_off;
+    r.m.fi64 = ctx->fi + ctx->nslot64() * c.geo_fi_off;
+    r.m.fj64 = ctx->fj + ctx->nslot64() * c.geo_fj_off;
     for (int d = 0; d < 2; ++d) {
         r.m.period_i[d] = c.cs.period_i[d];
         r.m.period_j[d] = c.cs.period_j[d];
@@ -360,7 +360,6 @@ template <class RF> void fill_rec(const hc_context* ctx, const CaseHost& c, int 
     r.N = c.N;
     r.cell_off = c.cell_off;
     r.bref_off = c.bref_off;
-    r.tiles_j = c.tiles_j[k];
 }
 
 // bitwise equality of two cases' device geometry (cells and face slots)
@@ -379,7 +378,7 @@ bool same_geometry(const GeomOutput& a, const GeomOutput& b)
 // (the part a single-case launch covers, from tile0).
 int build_tiles(hc_context* ctx)
 {
-    const TileShape* shapes = tile_shapes(ctx->precision == HC_PRECISION_MIXED, ctx->cs.law, ctx->cs.flux);
+    const TileShape* shapes = tile_shapes(ctx->precision == HC_PRECISION_MIXED, ctx->cs.law, ctx->cs.flux, ctx->fused);
     const int nc = (int)ctx->cases.size();
     for (int k = 0; k < NTILECFG; ++k) {
         long long nt = 0;
@@ -393,25 +392,29 @@ int build_tiles(hc_context* ctx)
         if (2 * nt > (1LL << 31) - 1) return fail(ctx, HC_ERR_ARG, "too many tiles");
         std::vector<TileRef> tab;
         tab.reserve((size_t)(2 * nt));
+        auto add = [&](int ci, int lt) {
+            const int tj = ctx->cases[ci].tiles_j[k];
+            tab.push_back(TileRef{ci, lt, (lt / tj) * shapes[k].ti, (lt % tj) * shapes[k].tj});
+        };
         if (ctx->interleave) {
             std::vector<std::vector<int>> members(nc);   // cases of each group, keyed by its first case
             for (int ci = 0; ci < nc; ++ci) members[ctx->cases[ci].geo].push_back(ci);
             for (int g = 0; g < nc; ++g)
                 for (int lt = 0; lt < ctx->cases[g].ntiles[k] && !members[g].empty(); ++lt)
-                    for (int ci : members[g]) tab.push_back(TileRef{ci, lt});
+                    for (int ci : members[g]) add(ci, lt);
         } else {
             for (int ci = 0; ci < nc; ++ci)
-                for (int lt = 0; lt < ctx->cases[ci].ntiles[k]; ++lt) tab.push_back(TileRef{ci, lt});
+                for (int lt = 0; lt < ctx->cases[ci].ntiles[k]; ++lt) add(ci, lt);
         }
         for (int ci = 0; ci < nc; ++ci) {
             ctx->cases[ci].tile0[k] = (int)tab.size();
-            for (int lt = 0; lt < ctx->cases[ci].ntiles[k]; ++lt) tab.push_back(TileRef{ci, lt});
+            for (int lt = 0; lt < ctx->cases[ci].ntiles[k]; ++lt) add(ci, lt);
         }
         std::vector<CaseRec<double>> r64(nc);
         std::vector<CaseRec<float>> r32(nc);
         for (int ci = 0; ci < nc; ++ci) {
-            fill_rec(ctx, ctx->cases[ci], k, r64[ci]);
-            fill_rec(ctx, ctx->cases[ci], k, r32[ci]);
+            fill_rec(ctx, ctx->cases[ci], r64[ci]);
+            fill_rec(ctx, ctx->cases[ci], r32[ci]);
         }
         free_dev(ctx->rec64[k]);
         free_dev(ctx->rec32[k]);
@@ -434,6 +437,9 @@ int build_layout(hc_context* ctx)
     if (ctx->cases.empty()) return fail(ctx, HC_ERR_STATE, "no case");
     ctx->cs = ctx->cases[0].cs;
     ctx->nv = ctx->cs.law == HC_LAW_EULER ? 4 : 3;
+    // a fixed step is the form that is differentiated (hc_adjoint.cpp): it keeps the reference's order,
+    // since the derivative of a limiter at slopes that almost vanish depends on their last bits
+    ctx->fused = fused_euler(ctx->cs.law, ctx->cs.flux) && ctx->cs.dt_mode != HC_DT_FIXED;
     ctx->nslots = make_rk_plans(ctx->cs.nstages, ctx->cs.alpha, ctx->cs.beta, ctx->plans);
     const int nv = ctx->nv;
     const int nc = (int)ctx->cases.size();
@@ -479,8 +485,9 @@ int build_layout(hc_context* ctx)
     HC_HIP(hipMalloc(&ctx->cvol, gN * sizeof(double)));
     HC_HIP(hipMalloc(&ctx->ccx, gN * sizeof(double)));
     HC_HIP(hipMalloc(&ctx->ccy, gN * sizeof(double)));
-    HC_HIP(hipMalloc(&ctx->fi, NSLOT * gfi * sizeof(double)));
-    HC_HIP(hipMalloc(&ctx->fj, NSLOT * gfj * sizeof(double)));
+    const long long nslot = ctx->nslot64();
+    HC_HIP(hipMalloc(&ctx->fi, nslot * gfi * sizeof(double)));
+    HC_HIP(hipMalloc(&ctx->fj, nslot * gfj * sizeof(double)));
     HC_HIP(hipMalloc(&ctx->fi32, NSLOT * gfi * sizeof(float)));
     HC_HIP(hipMalloc(&ctx->fj32, NSLOT * gfj * sizeof(float)));
     for (int ci = 0; ci < nc; ++ci) {
@@ -489,10 +496,17 @@ int build_layout(hc_context* ctx)
             HC_HIP(hipMemcpy(ctx->cvol + c.geo_cell_off, c.g.cvol.data(), c.N * sizeof(double), hipMemcpyHostToDevice));
             HC_HIP(hipMemcpy(ctx->ccx + c.geo_cell_off, c.g.ccx.data(), c.N * sizeof(double), hipMemcpyHostToDevice));
             HC_HIP(hipMemcpy(ctx->ccy + c.geo_cell_off, c.g.ccy.data(), c.N * sizeof(double), hipMemcpyHostToDevice));
-            HC_HIP(hipMemcpy(ctx->fi + NSLOT * c.geo_fi_off, c.g.fi.data(), c.g.fi.size() * sizeof(double),
-                             hipMemcpyHostToDevice));
-            HC_HIP(hipMemcpy(ctx->fj + NSLOT * c.geo_fj_off, c.g.fj.data(), c.g.fj.size() * sizeof(double),
-                             hipMemcpyHostToDevice));
+            double* fi = ctx->fi + nslot * c.geo_fi_off;
+            double* fj = ctx->fj + nslot * c.geo_fj_off;
+            HC_HIP(hipMemcpy(fi, c.g.fi.data(), c.g.fi.size() * sizeof(double), hipMemcpyHostToDevice));
+            HC_HIP(hipMemcpy(fj, c.g.fj.data(), c.g.fj.size() * sizeof(double), hipMemcpyHostToDevice));
+            if (ctx->fused) {
+                std::vector<double> w;
+                directional_weights(c.g.fi, c.nfi, w);
+                HC_HIP(hipMemcpy(fi + NSLOT * c.nfi, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice));
+                directional_weights(c.g.fj, c.nfj, w);
+                HC_HIP(hipMemcpy(fj + NSLOT * c.nfj, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice));
+            }
             std::vector<float> f32;
             fp32_slots(c.g.fi, c.nfi, f32);
             HC_HIP(hipMemcpy(ctx->fi32 + NSLOT * c.geo_fi_off, f32.data(), f32.size() * sizeof(float),
@@ -539,7 +553,11 @@ int build_layout(hc_context* ctx)
     HC_HIP(hipMemcpy(ctx->chunks, ch.data(), ch.size() * sizeof(UpdChunk), hipMemcpyHostToDevice));
     ctx->nchunks = (int)ch.size();
     ctx->uni_ok = true;
-    for (const auto& c : ctx->cases) ctx->uni_ok = ctx->uni_ok && c.uniform;
+    ctx->wide = false;
+    for (const auto& c : ctx->cases) {
+        ctx->uni_ok = ctx->uni_ok && c.uniform;
+        ctx->wide = ctx->wide || 8 * std::max(c.nfi, c.nfj) >= (1LL << 32) || std::max(c.ni, c.nj) >= (1 << 24) - 1;
+    }
     ctx->have_case = true;
     return HC_OK;
 }
@@ -553,6 +571,8 @@ template <class RF> LaunchArgs<RF> launch_args(hc_context* ctx)
     L.tile_base = 0;
     L.ntiles = ctx->ntiles[ctx->tile_cfg];
     L.nslots = ctx->nslots;
+    L.fused = ctx->fused && ctx->precision == HC_PRECISION_FP64 ? 1 : 0;
+    L.wide = ctx->wide ? 1 : 0;
     L.vscale = ctx->cs.vscale;
     L.pscale = ctx->cs.pscale;
     L.limiter = ctx->cs.limiter;

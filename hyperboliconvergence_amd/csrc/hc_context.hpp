@@ -81,6 +81,9 @@ struct hc_context {
     // tile shape: fixed index, or -1 to time every shape on the first steps and keep the fastest
     int tile_mode = -1;
     int tile_cfg = 0;
+    bool fused = false;            // FP64 runs the fused Euler tile (hc_fused.hpp)
+    long long nslot64() const { return fused ? hc::NSLOT_FUSED : hc::NSLOT; }   // planes of the FP64 face slots
+    bool wide = false;             // some case's planes pass 32-bit byte offsets (LaunchArgs::wide)
     bool uni_ok = false;           // every case has uniform geometry
     bool uni_enable = true;        // use the uniform-geometry kernels when uni_ok (hc_set_uniform_geometry)
     bool tuned = false;

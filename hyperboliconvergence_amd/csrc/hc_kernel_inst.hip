@@ -2,6 +2,10 @@
 // -DHC_LAW=<0|1> -DHC_BASIS=<0|1> -DHC_FLUX=<0..5> -DHC_PREC=<64|32>, in every tile shape
 // of its precision.  The FP64 objects are compiled with -ffp-contract=off (bit-faithful
 // arithmetic), the mixed ones with contraction allowed.
+#if defined(HC_PREC) && HC_PREC == 32
+#define HC_MIXED_OBJECT
+#endif
+#include "hc_fused.hpp"
 #include "hc_launch.hpp"
 
 #if !defined(HC_LAW) || !defined(HC_BASIS) || !defined(HC_FLUX) || !defined(HC_PREC)
@@ -13,21 +17,36 @@
 #define HC_UNAME3(L, B, P) hc_upd_L##L##_B##B##_P##P
 #define HC_UNAME(L, B, P) HC_UNAME3(L, B, P)
 
+#ifndef HC_FWPE
+#define HC_FWPE 5
+#endif
 #if HC_PREC == 64
 using RF = double;
 #else
 using RF = float;
 #endif
 
-// UNI: the uniform-geometry kernel of the shape; centre staging has nothing to stage there, so a
-// shape that differs from another only by it shares that shape's kernel
-template <int K, int UNI> static hipError_t launch_shape(const hc::LaunchArgs<RF>& L, hipStream_t st)
+template <class T, int WPE, class A> static hipError_t launch(const A& L, hipStream_t st)
 {
-    constexpr hc::TileShape S = hc::tile_shapes(HC_PREC == 32, HC_LAW, HC_FLUX)[K];
-    constexpr int CST = UNI ? 0 : S.cst;
-    hipLaunchKernelGGL((hc::k_stage<HC_LAW, HC_BASIS, HC_FLUX, RF, S.ti, S.tj, S.nt, CST, S.gpf, UNI>), dim3(L.ntiles),
-                       dim3(S.nt), 0, st, L);
+    hipLaunchKernelGGL((hc::k_stage<T, RF, WPE>), dim3(L.ntiles), dim3(T::NT), 0, st, L);
     return hipGetLastError();
+}
+
+// UNI: the uniform-geometry kernel of the shape
+template <int K, int UNI, class A> static hipError_t launch_shape(const A& L, hipStream_t st)
+{
+    if constexpr (HC_PREC == 64 && hc::fused_euler(HC_LAW, HC_FLUX)) {
+        constexpr hc::TileShape S = hc::TILESF[K];
+        // 64-bit offsets only where a plane needs them, and then without the uniform-geometry variant
+        if (L.fused && L.wide)
+            return launch<hc::FusedTile<HC_BASIS, HC_FLUX, S.ti, S.tj, S.nt, unsigned long long, 0>, 4>(L, st);
+        if (L.fused) return launch<hc::FusedTile<HC_BASIS, HC_FLUX, S.ti, S.tj, S.nt, unsigned, UNI>, HC_FWPE>(L, st);
+    }
+    // centre staging has nothing to stage on uniform geometry, so a shape that differs from another
+    // only by it shares that shape's kernel
+    constexpr hc::TileShape S = hc::tile_shapes(HC_PREC == 32, HC_LAW, HC_FLUX, false)[K];
+    return launch<hc::StageTile<HC_LAW, HC_BASIS, HC_FLUX, RF, S.ti, S.tj, S.nt, UNI ? 0 : S.cst, S.gpf, UNI>,
+                  (S.gpf != 0 ? 4 : 1)>(L, st);
 }
 
 hipError_t HC_NAME(HC_LAW, HC_BASIS, HC_FLUX, HC_PREC)(const hc::LaunchArgs<RF>& L, int cfg, int uni, hipStream_t st)

@@ -43,6 +43,9 @@ constexpr int FS_CY = FS_DR;
 // factors in place of the factors (two per side)
 constexpr int FS_WL0 = FS_FL0, FS_WL1 = FS_FL1, FS_WR0 = FS_FR0, FS_WR1 = FS_FR1;
 
+// the GPU's FP64 slots of a fused context (hc_fused.hpp) are followed by the same weights in FP64
+enum { FS_XL0 = NSLOT, FS_XL1, FS_XR0, FS_XR1, NSLOT_FUSED };
+
 // status bits returned through the C-ABI
 enum StatusBits : unsigned int {
     ST_NONFINITE = 1u,     // non-finite state after an update
@@ -188,6 +191,7 @@ template <int LAW, int BASIS, int FLUX, class RF, int TI, int TJ, int NTHR = TI 
           int UNI = 0>
 struct StageTile {
     static constexpr int NV = LawTraits<LAW>::nv;
+    static constexpr int TILE_I = TI, TILE_J = TJ;
     static constexpr int NC = TI * TJ;   // cells of the tile
     static constexpr int NT = NTHR;      // threads of the work-group
     static_assert(NT >= NC, "one thread per cell at least");
@@ -625,6 +629,7 @@ struct StageTile {
     // made per flux for all tile configurations alike: a cell phase of another shape in some of them
     // could contract the update differently, and cases would then depend on the tile shape in the
     // last bits.
+    static constexpr bool REREAD = UNI == 0;   // case parameters read again per phase (k_stage)
     static constexpr bool LPF = (GPF != 0 && !CPF) || (sizeof(RF) == sizeof(float) && FLUX != FLUX_AUSMPUP);
     static constexpr bool PF = CPF || LPF;
     struct CellIn {
@@ -808,7 +813,6 @@ template <class RF> struct CaseRec {
     long long N;          // cells of the case
     long long cell_off;   // first cell of the case in the packed per-cell arrays
     long long bref_off;   // first boundary-reference row of the case
-    int tiles_j;          // tiles along j in the record's tile shape
 };
 
 // One entry of a context's tile table: the case and the tile within the case (row-major over the
@@ -818,6 +822,7 @@ template <class RF> struct CaseRec {
 struct TileRef {
     int ci;
     int lt;
+    int i0, j0;   // the tile's first cell
 };
 
 template <class RF> struct LaunchArgs {
@@ -826,6 +831,8 @@ template <class RF> struct LaunchArgs {
     int tile_base;          // first entry of the launch in the table
     int ntiles;             // tiles of the launch
     int nslots;
+    int fused;            // the context runs the fused Euler tile (hc_fused.hpp)
+    int wide;             // a plane of cells or faces of some case passes its 32-bit byte offsets
     int vscale, pscale, limiter;
     int mode, dt_mode, stage, reset_max;
     int keep_res;         // fused stages: also store the stage's residual in res_out (stage 0 of a step)
@@ -913,22 +920,19 @@ static_assert(MAXSPREAD == 64, "one slot per lane of a wavefront");
 #define HC_STAGE_OCCUPANCY
 #endif
 
-// The prefetching configurations hold the prefetched values across the metric phase: at least 4
-// waves per SIMD keeps them within 128 VGPRs (the AUSM+up FP64 kernel would otherwise take 129
-// and drop to 3 waves)
-template <int LAW, int BASIS, int FLUX, class RF, int TI, int TJ, int NTHR, int CST, int GPF, int UNI = 0>
-__global__ void __launch_bounds__(NTHR) HC_STAGE_OCCUPANCY __attribute__((amdgpu_waves_per_eu(GPF != 0 ? 4 : 1)))
-k_stage(LaunchArgs<RF> L)
+// T: the tile (StageTile, or FusedTile of hc_fused.hpp).  WPE: the occupancy asked for, in waves per SIMD.
+// The prefetching configurations hold the prefetched values across the metric phase: at least 4 keeps
+// them within 128 VGPRs.
+template <class T, class RF, int WPE>
+__global__ void __launch_bounds__(T::NT) HC_STAGE_OCCUPANCY __attribute__((amdgpu_waves_per_eu(WPE))) k_stage(LaunchArgs<RF> L)
 {
-    using T = StageTile<LAW, BASIS, FLUX, RF, TI, TJ, NTHR, CST, GPF, UNI>;
     __shared__ typename T::Smem s;
     const int tid = threadIdx.x;
     // XCD-aware tile order: consecutive work-group ids are dealt round-robin to the
     // 8 XCDs, so give each XCD a contiguous band of tiles (shared halos stay in one L2)
     const TileRef tr = L.tiles[L.tile_base + xcd_tile(blockIdx.x, L.ntiles)];
-    const int ci = tr.ci, lt = tr.lt;
+    const int ci = tr.ci, lt = tr.lt, i0 = tr.i0, j0 = tr.j0;
     const CaseRec<RF>& c = L.cases[ci];
-    const int i0 = (lt / c.tiles_j) * TI, j0 = (lt % c.tiles_j) * TJ;
     // The case's parameters (18 array pointers, species, Runge-Kutta plan) held from the first
     // phase to the last exceed the scalar register file, and the kernels then spill them into
     // vector-register lanes (about 110 lane moves per wavefront).  Instead, a group of phases reads
@@ -937,7 +941,7 @@ k_stage(LaunchArgs<RF> L)
     // of the previous group die at its barrier: the general-geometry kernels read them for the
     // face phase and again for the cell phase, the uniform-geometry kernels once more for the cell
     // phase only (a read for their face phase costs them vector registers and time).
-    auto args = [&](bool reread = UNI == 0) -> StageArgs<RF> {
+    auto args = [&](bool reread = T::REREAD) -> StageArgs<RF> {
         if (!reread) {
             return case_args<RF, T::NV>(L, c, ci);
         } else {
@@ -970,11 +974,13 @@ k_stage(LaunchArgs<RF> L)
     double red;
     const StageArgs<RF> a = args(true);
     T::cells(a, s, i0, j0, tid, flag, red, cin);
-    // reductions: the status bits; for global-dt stage 0 also max(lambda/vol), over the
-    // work-group and into the tile's slot (mode is uniform over the grid: the barrier is too)
-    const double m = wave_max(red);
-    const unsigned int f = wave_or(flag);
+    // reductions: the status bits, which are almost never set, where some lane has one; for global-dt
+    // stage 0 also max(lambda/vol), over the work-group and into the tile's slot (mode is uniform over
+    // the grid: the barrier is too)
+    unsigned int f = 0;
+    if (__any(flag != 0)) f = wave_or(flag);
     if (a.mode == MODE_GLOBAL_STAGE0) {
+        const double m = wave_max(red);
         static_assert(T::NT % 64 == 0, "whole wavefronts");
         __shared__ unsigned long long wm[T::NT / 64];
         __shared__ unsigned int wf[T::NT / 64];

@@ -29,11 +29,16 @@ struct TileShape {
 // AUSM+up take larger tiles: 8x32 (552 faces), 7x32 (487 faces, two per lane) on 256 lanes, or
 // 7x16.
 constexpr int NTILECFG = 3;
-constexpr TileShape TILES64[NTILECFG] = {{4, 32, 256, 0, 0}, {7, 16, 256, 0, 1}, {7, 16, 256, 1, 1}};
+constexpr TileShape TILES64[NTILECFG] = {{7, 16, 256, 1, 1}, {7, 16, 256, 0, 1}, {4, 32, 256, 0, 0}};
 constexpr TileShape TILES32[NTILECFG] = {{8, 32, 256, 0, 0}, {7, 32, 256, 0, 0}, {7, 16, 256, 0, 0}};
 
-constexpr const TileShape* tile_shapes(bool mixed, int law, int flux)
+// Euler in FP64 (FusedTile): one face per lane, i-faces in whole wavefronts, centres staged and face
+// slots prefetched in all of them.
+constexpr TileShape TILESF[NTILECFG] = {{7, 16, 256, 1, 1}, {7, 8, 128, 1, 1}, {15, 16, 512, 1, 1}};
+
+constexpr const TileShape* tile_shapes(bool mixed, int law, int flux, bool fused)
 {
+    if (!mixed && fused) return TILESF;
     return (!mixed || mixed_wide(law, flux)) ? TILES64 : TILES32;
 }
 

@@ -5,6 +5,7 @@
 // buffer rotation and Runge-Kutta plans as the C-ABI.  Tests use it to check the
 // kernels' arithmetic and LDS indexing against the oracle without a GPU.  It is
 // never part of the product library.
+#include "hc_fused.hpp"
 #include "hc_geom.hpp"
 #include "hc_stage.hpp"
 #include "hc_tiles.hpp"
@@ -82,10 +83,9 @@ template <class RF> StageArgs<RF> args_of(Emu& e)
 // uniform-geometry kernels (UNI) when the case allows them, selected with emu_set_uniform_geometry
 int g_uniform = 0;
 
-template <int LAW, int BASIS, int FLUX, class RF, int TI, int TJ, int NT, int CST, int GPF, int UNI>
-void run_stage_t(const StageArgs<RF>& a)
+template <class T, class RF> void run_tiles(const StageArgs<RF>& a)
 {
-    using T = StageTile<LAW, BASIS, FLUX, RF, TI, TJ, NT, CST, GPF, UNI>;
+    constexpr int TI = T::TILE_I, TJ = T::TILE_J;
     const int tiles_i = (a.m.ni + TI - 1) / TI, tiles_j = (a.m.nj + TJ - 1) / TJ;
     const int ntiles = tiles_i * tiles_j;
     auto sp = std::make_unique<typename T::Smem>();
@@ -118,7 +118,35 @@ void run_stage_t(const StageArgs<RF>& a)
     if (a.reset_max) *a.maxslot = dbl_bits(DBL_MIN);
 }
 
+template <int LAW, int BASIS, int FLUX, class RF, int TI, int TJ, int NT, int CST, int GPF, int UNI>
+void run_stage_t(const StageArgs<RF>& a)
+{
+    run_tiles<StageTile<LAW, BASIS, FLUX, RF, TI, TJ, NT, CST, GPF, UNI>>(a);
+}
+
 bool g_case_uniform = false;
+
+// the fused Euler tile (hc_fused.hpp) in FP64: 1 with 32-bit offsets, 2 with 64-bit ones
+int g_fused = 0;
+
+template <int BASIS, int FLUX, int K> void run_fused_flux(const StageArgs<double>& a)
+{
+    constexpr TileShape S = TILESF[K];
+    if (g_uniform && g_case_uniform) run_tiles<FusedTile<BASIS, FLUX, S.ti, S.tj, S.nt, unsigned, 1>>(a);
+    else if (g_fused == 2) run_tiles<FusedTile<BASIS, FLUX, S.ti, S.tj, S.nt, unsigned long long, 0>>(a);
+    else run_tiles<FusedTile<BASIS, FLUX, S.ti, S.tj, S.nt, unsigned, 0>>(a);
+}
+
+template <int BASIS, int K> void run_fused(int flux, const StageArgs<double>& a)
+{
+    switch (flux) {
+    case 0: run_fused_flux<BASIS, 0, K>(a); break;
+    case 1: run_fused_flux<BASIS, 1, K>(a); break;
+    case 4: run_fused_flux<BASIS, 4, K>(a); break;
+    case 5: run_fused_flux<BASIS, 5, K>(a); break;
+    default: run_fused_flux<BASIS, 6, K>(a); break;
+    }
+}
 
 template <int LAW, int BASIS, int FLUX, class RF, int TI, int TJ, int NT, int CST, int GPF>
 void run_stage(const StageArgs<RF>& a)
@@ -174,7 +202,10 @@ int g_tile_cfg = 0;
 template <int K> void stage_shape(Emu& e, StageArgs<double>& a64, StageArgs<float>& a32)
 {
     constexpr TileShape S64 = TILES64[K], S32 = TILES32[K];
-    if (e.precision != HC_PRECISION_MIXED) dispatch_stage<double, S64.ti, S64.tj, S64.nt, S64.cst, S64.gpf>(e.cs, a64);
+    if (g_fused && e.precision != HC_PRECISION_MIXED && e.cs.law == HC_LAW_EULER) {
+        if (e.cs.basis == HC_BASIS_CONSERVED) run_fused<0, K>(e.cs.flux, a64);
+        else run_fused<1, K>(e.cs.flux, a64);
+    } else if (e.precision != HC_PRECISION_MIXED) dispatch_stage<double, S64.ti, S64.tj, S64.nt, S64.cst, S64.gpf>(e.cs, a64);
     else if (mixed_wide(e.cs.law, e.cs.flux))
         dispatch_stage<float, S64.ti, S64.tj, S64.nt, S64.cst, S64.gpf>(e.cs, a32);
     else dispatch_stage<float, S32.ti, S32.tj, S32.nt, S32.cst, S32.gpf>(e.cs, a32);
@@ -208,6 +239,11 @@ int setup(Emu& e, const hc_case_desc* cs, int ni, int nj, const double* nodes, c
     g_case_uniform = uniform_geometry(gin, e.g);
     fp32_slots(e.g.fi, (long long)(ni + 1) * nj, e.fi32);
     fp32_slots(e.g.fj, (long long)ni * (nj + 1), e.fj32);
+    std::vector<double> w;   // the weight slots of a fused context
+    directional_weights(e.g.fi, (long long)(ni + 1) * nj, w);
+    e.g.fi.insert(e.g.fi.end(), w.begin(), w.end());
+    directional_weights(e.g.fj, (long long)ni * (nj + 1), w);
+    e.g.fj.insert(e.g.fj.end(), w.begin(), w.end());
     const long long N = (long long)ni * nj;
     for (auto& b : e.q) b.assign((size_t)e.nv * N, 0.0);
     for (long long c = 0; c < N; ++c)
@@ -238,6 +274,14 @@ int emu_set_tile_config(int cfg)
 {
     if (cfg < 0 || cfg >= NTILECFG) return -1;
     g_tile_cfg = cfg;
+    return 0;
+}
+
+// 0: the stage tiles in the reference's order; 1 / 2: the fused Euler tile with 32- / 64-bit offsets
+int emu_set_fused(int mode)
+{
+    if (mode < 0 || mode > 2) return -1;
+    g_fused = mode;
     return 0;
 }
 

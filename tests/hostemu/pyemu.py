@@ -31,6 +31,7 @@ def lib():
         _L.emu_geometry.argtypes = [P, i, i, P, P, P, P, P]
         _L.emu_set_tile_config.argtypes = [i]
         _L.emu_set_uniform_geometry.argtypes = [i]
+        _L.emu_set_fused.argtypes = [i]
         _L.emu_tangent_residual.argtypes = [P, i, i, P, P, P, P, P, C.c_double, P, P]
         _L.emu_adjoint_residual.argtypes = [P, i, i, P, P, P, P, P, P, P]
     return _L
@@ -45,6 +46,12 @@ def set_uniform_geometry(enable):
     """1: emulate the uniform-geometry kernels on cases that allow them; returns whether the last
     case set up allowed them."""
     return bool(lib().emu_set_uniform_geometry(int(enable)))
+
+
+def set_fused(mode):
+    """0: stage tiles in the reference's order (FP64); 1 / 2: the fused Euler tile with 32- / 64-bit
+    offsets."""
+    assert lib().emu_set_fused(int(mode)) == 0
 
 
 def _p(a):
