@@ -175,18 +175,19 @@ template <int BASIS, int FLUX, int TI, int TJ, int NTHR, class Off, int UNI> str
         g.wr1 = slot(b + FS_XR1 * nf, o);
     }
 
-    // the slots of the lane's face, loaded with the tile
+    // the slots of the lane's face, loaded with the tile; lanes and faces beyond the tile or the mesh take
+    // the last ones, so that every lane's registers are written
     HC_HD static void prefetch(const StageArgs<double>& a, int i0, int j0, int tid, Geo& g)
     {
-        if (UNI || tid >= NF) return;
-        const bool isi = kind_i(tid);
+        if (UNI) return;
+        const int k = tid < NF ? tid : NF - 1;
+        const bool isi = kind_i(k);
         int li, lj;
-        pos(tid, isi, li, lj);
-        int l = isi ? i0 + li : j0 + lj;
-        const int t = isi ? j0 + lj : i0 + li;
-        const int lmax = isi ? a.m.ni : a.m.nj;
-        if (l > lmax || t >= (isi ? a.m.nj : a.m.ni)) return;
-        if (isi ? a.m.per_i : a.m.per_j) l = l == lmax ? 0 : l;   // the wrap face is held on node line 0
+        pos(k, isi, li, lj);
+        const int lmax = isi ? a.m.ni : a.m.nj, tmax = (isi ? a.m.nj : a.m.ni) - 1;
+        int l = isi ? i0 + li : j0 + lj, t = isi ? j0 + lj : i0 + li;
+        l = l < lmax ? l : (isi ? a.m.per_i : a.m.per_j) ? 0 : lmax;   // the wrap face is held on node line 0
+        t = t < tmax ? t : tmax;
         slots(isi ? a.m.fi : a.m.fj, isi ? a.m.nfi : a.m.nfj, isi ? offset(l, a.m.nj, t) : offset(t, a.m.nj + 1, l), g);
     }
 

@@ -17,9 +17,6 @@
 #define HC_UNAME3(L, B, P) hc_upd_L##L##_B##B##_P##P
 #define HC_UNAME(L, B, P) HC_UNAME3(L, B, P)
 
-#ifndef HC_FWPE
-#define HC_FWPE 5
-#endif
 #if HC_PREC == 64
 using RF = double;
 #else
@@ -40,7 +37,7 @@ template <int K, int UNI, class A> static hipError_t launch_shape(const A& L, hi
         // 64-bit offsets only where a plane needs them, and then without the uniform-geometry variant
         if (L.fused && L.wide)
             return launch<hc::FusedTile<HC_BASIS, HC_FLUX, S.ti, S.tj, S.nt, unsigned long long, 0>, 4>(L, st);
-        if (L.fused) return launch<hc::FusedTile<HC_BASIS, HC_FLUX, S.ti, S.tj, S.nt, unsigned, UNI>, HC_FWPE>(L, st);
+        if (L.fused) return launch<hc::FusedTile<HC_BASIS, HC_FLUX, S.ti, S.tj, S.nt, unsigned, UNI>, 5>(L, st);
     }
     // centre staging has nothing to stage on uniform geometry, so a shape that differs from another
     // only by it shares that shape's kernel
