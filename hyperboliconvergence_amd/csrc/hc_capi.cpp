@@ -684,6 +684,14 @@ void drain_events(hc_context* ctx)
     ctx->ev_pending.clear();
 }
 
+// Whether a step folds its stage-0 update into stage 1 (StageArgs::beta_in): the max slots that stage 1
+// then reads are re-armed by a later stage, so tables of one and two stages keep the kernel, and so do
+// planes beyond 32-bit offsets, which have no such variant
+bool folds(const hc_context* ctx)
+{
+    return ctx->cs.dt_mode == HC_DT_GLOBAL && ctx->cs.nstages >= 3 && !ctx->wide;
+}
+
 // the launches of one time step of every case (timestepping/rungeKutta.h:97-164)
 int enqueue_step(hc_context* ctx)
 {
@@ -700,6 +708,7 @@ int enqueue_step(hc_context* ctx)
         bufB = ctx->q[(ctx->cur + 2) % 3];
     }
     LaunchArgs<double> L = launch_args<double>(ctx);
+    const bool fold = folds(ctx);
     const double* in = q0;
     for (int s = 0; s < ns; ++s) {
         double* out;
@@ -714,9 +723,11 @@ int enqueue_step(hc_context* ctx)
         L.reset_max = (global && ns >= 2 && s == ns - 1) ? 1 : 0;
         L.mode = (global && s == 0) ? MODE_GLOBAL_STAGE0 : MODE_FUSED;
         L.keep_res = (ctx->keep_res && s == 0) ? 1 : 0;
+        L.upd_in = fold && s == 1 ? 1 : 0;
+        L.beta_in = ctx->plans[0].beta;
         hipError_t e = timed(ctx, 0, [&] { return launch_stage(ctx, L); });
         if (e != hipSuccess) return hipfail(ctx, e, "stage kernel launch");
-        if (global && s == 0) {
+        if (global && s == 0 && !fold) {
             e = timed(ctx, 1, [&] { return launch_update(ctx, L); });
             if (e != hipSuccess) return hipfail(ctx, e, "update kernel launch");
         }
@@ -1247,7 +1258,7 @@ int hc_step(hc_context* ctx, int nsteps)
     if (r0) {
         hipEvent_t r1 = take_event(ctx);
         (void)hipEventRecord(r1, ctx->stream);
-        const double upd = ctx->cs.dt_mode == HC_DT_GLOBAL ? 1.0 : 0.0;
+        const double upd = ctx->cs.dt_mode == HC_DT_GLOBAL && !folds(ctx) ? 1.0 : 0.0;
         ctx->ev_pending.push_back({r0, r1, double(nsteps) * ctx->cs.nstages, double(nsteps) * upd, 2});
     }
     if (ctx->profiling == 1) drain_events(ctx);

@@ -21,8 +21,9 @@ namespace hc {
 
 // Off: byte offset into a plane of cells or faces: 32 bits where every plane is below 4 GiB, so that
 // a load is a scalar base and one vector register; 64 bits otherwise.
-template <int BASIS, int FLUX, int TI, int TJ, int NTHR, class Off, int UNI> struct FusedTile {
+template <int BASIS, int FLUX, int TI, int TJ, int NTHR, class Off, int UNI, int FOLD = 0> struct FusedTile {
     static constexpr int NV = 4, TILE_I = TI, TILE_J = TJ;
+    static constexpr bool FOLDS = FOLD != 0;
     static constexpr int NC = TI * TJ, NT = NTHR;
     static constexpr int QH = TI + 4, QW = TJ + 4;   // state tile with a 2-cell halo
     static constexpr int MH = TI + 2, MW = TJ + 2;   // metric ring with a 1-cell halo
@@ -92,14 +93,48 @@ template <int BASIS, int FLUX, int TI, int TJ, int NTHR, class Off, int UNI> str
         dy = gc[QH * QW + pr] - (gc[QH * QW + pl] - (wrap ? py : 0.0));
     }
 
-    HC_HD static void load(const StageArgs<double>& a, Smem& s, int i0, int j0, int tid)
+    HC_HD static bool folded(const StageArgs<double>& a)
+    {
+#if defined(__HIP_DEVICE_COMPILE__)
+        return FOLDS;
+#else
+        return a.fold_in != 0;
+#endif
+    }
+
+    // updated() (hc_stage.hpp) with a cheaper finiteness check: 0 x finite = 0, and an infinity or NaN in
+    // any variable leaves NaN
+    HC_HD static void advance(const StageArgs<double>& a, const double* q0, const double* Rt, double fac, double* q1,
+                              unsigned int& flag)
+    {
+        double qc[NV], nan = 0.0;
+        to_conserved<double, LAW_EULER, BASIS>(a.sp, q0, qc);
+        for (int v = 0; v < NV; ++v) qc[v] = qc[v] + Rt[v] * fac;
+        from_conserved<double, LAW_EULER, BASIS>(a.sp, qc, q1);
+        for (int v = 0; v < NV; ++v) nan = hc_fma(0.0, q1[v], nan);
+        if (nan != nan) flag |= ST_NONFINITE;
+        if (!(q1[2] > 0.0) || (BASIS == BASIS_PRIMITIVE && !(q1[3] > 0.0))) flag |= ST_NONPHYSICAL;
+    }
+
+    HC_HD static void load(const StageArgs<double>& a, Smem& s, int i0, int j0, int tid, unsigned int& flag)
     {
         for (int k = tid; k < QH * QW; k += NT) {
             const int li = k / QW, lj = k % QW;
             const int gi = halo(i0 - 2 + li, a.m.ni, a.m.per_i);
             const int gj = halo(j0 - 2 + lj, a.m.nj, a.m.per_j);
             const Off o = offset(gi, a.m.nj, gj);
-            for (int v = 0; v < NV; ++v) s.q[v][li][lj] = at(a.q_in + v * a.N, o);
+            if (folded(a)) {
+                double q0[NV], Rt[NV], q1[NV];
+                for (int v = 0; v < NV; ++v) {
+                    q0[v] = at(a.q0 + v * a.N, o);
+                    Rt[v] = at(a.tmp + v * a.N, o);
+                }
+                const double vol = UNI ? uniform(a.m.cvol) : at(a.m.cvol, o);
+                advance(a, q0, Rt, hc_div(a.beta_in * a.dt_in, vol), q1, flag);
+                for (int v = 0; v < NV; ++v) s.q[v][li][lj] = q1[v];
+            } else {
+                for (int v = 0; v < NV; ++v) s.q[v][li][lj] = at(a.q_in + v * a.N, o);
+            }
             if constexpr (!UNI) {
                 s.gc[0][li][lj] = at(a.m.ccx, o);
                 s.gc[1][li][lj] = at(a.m.ccy, o);
@@ -373,7 +408,7 @@ template <int BASIS, int FLUX, int TI, int TJ, int NTHR, class Off, int UNI> str
         }
         double fac;
         if (a.dt_mode == 0) {
-            fac = hc_div(p.beta * a.dtslot[0], ci.vol);
+            fac = hc_div(p.beta * (folded(a) ? a.dt_in : a.dtslot[0]), ci.vol);
         } else if (a.dt_mode == 2) {
             fac = hc_div(p.beta * a.cfl, ci.vol);   // fixed step: cfl holds dt
         } else {
@@ -381,18 +416,9 @@ template <int BASIS, int FLUX, int TI, int TJ, int NTHR, class Off, int UNI> str
             if (a.stage == 0) put(a.lam0, o, lam);
             fac = hc_div(p.beta * a.cfl, l0);
         }
-        // q_out = S( C(q0) + R_tot*fac )   (spatial/eulerForwardUpdate.h:76-85)
-        double qc[NV], qn[NV];
-        to_conserved<double, LAW_EULER, BASIS>(a.sp, ci.q0, qc);
-        for (int v = 0; v < NV; ++v) qc[v] = qc[v] + Rt[v] * fac;
-        from_conserved<double, LAW_EULER, BASIS>(a.sp, qc, qn);
-        double nan = 0.0;   // 0 x finite = 0; an infinity or NaN anywhere leaves NaN
-        for (int v = 0; v < NV; ++v) {
-            put(a.q_out + v * a.N, o, qn[v]);
-            nan = hc_fma(0.0, qn[v], nan);
-        }
-        if (nan != nan) flag |= ST_NONFINITE;
-        if (!(qn[2] > 0.0) || (BASIS == BASIS_PRIMITIVE && !(qn[3] > 0.0))) flag |= ST_NONPHYSICAL;
+        double qn[NV];
+        advance(a, ci.q0, Rt, fac, qn, flag);
+        for (int v = 0; v < NV; ++v) put(a.q_out + v * a.N, o, qn[v]);
     }
 };
 

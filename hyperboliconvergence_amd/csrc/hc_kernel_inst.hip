@@ -37,13 +37,17 @@ template <int K, int UNI, class A> static hipError_t launch_shape(const A& L, hi
         // 64-bit offsets only where a plane needs them, and then without the uniform-geometry variant
         if (L.fused && L.wide)
             return launch<hc::FusedTile<HC_BASIS, HC_FLUX, S.ti, S.tj, S.nt, unsigned long long, 0>, 4>(L, st);
+        if (L.fused && L.upd_in)
+            return launch<hc::FusedTile<HC_BASIS, HC_FLUX, S.ti, S.tj, S.nt, unsigned, UNI, 1>, 5>(L, st);
         if (L.fused) return launch<hc::FusedTile<HC_BASIS, HC_FLUX, S.ti, S.tj, S.nt, unsigned, UNI>, 5>(L, st);
     }
     // centre staging has nothing to stage on uniform geometry, so a shape that differs from another
     // only by it shares that shape's kernel
     constexpr hc::TileShape S = hc::tile_shapes(HC_PREC == 32, HC_LAW, HC_FLUX, false)[K];
-    return launch<hc::StageTile<HC_LAW, HC_BASIS, HC_FLUX, RF, S.ti, S.tj, S.nt, UNI ? 0 : S.cst, S.gpf, UNI>,
-                  (S.gpf != 0 ? 4 : 1)>(L, st);
+    constexpr int WPE = S.gpf != 0 ? 4 : 1, CST = UNI ? 0 : S.cst;
+    if (L.upd_in)
+        return launch<hc::StageTile<HC_LAW, HC_BASIS, HC_FLUX, RF, S.ti, S.tj, S.nt, CST, S.gpf, UNI, 1>, WPE>(L, st);
+    return launch<hc::StageTile<HC_LAW, HC_BASIS, HC_FLUX, RF, S.ti, S.tj, S.nt, CST, S.gpf, UNI>, WPE>(L, st);
 }
 
 hipError_t HC_NAME(HC_LAW, HC_BASIS, HC_FLUX, HC_PREC)(const hc::LaunchArgs<RF>& L, int cfg, int uni, hipStream_t st)

@@ -85,8 +85,8 @@ enum StageMode { MODE_FUSED = 0, MODE_GLOBAL_STAGE0 = 1, MODE_RESIDUAL = 2 };
 // A case's max(lambda/vol) of global-dt stage 0 is reduced into MAXSPREAD slots, each on its own
 // 128-byte line (MAXSTRIDE words apart), one atomic per work-group on the slot of its tile index:
 // atomics on one address serialise (a 4096^2 grid has 524288 waves), atomics on 64 lines do not.
-// The update kernel takes the max of the slots with one load per lane of a wavefront.
-constexpr int MAXSPREAD = 64, MAXSTRIDE = 16;
+// The reader takes the max of the slots with one load per lane of a wavefront.
+constexpr int MAXSPREAD = 64, MAXSTRIDE = 2;
 
 // Accumulation plans of a Runge-Kutta table in the reference's (alpha, beta) form
 // (ode.h:87-105): one accumulator per later row with a non-zero coefficient
@@ -128,6 +128,14 @@ template <class RF> struct StageArgs {
     int bc[4];
     int mode, dt_mode, stage, reset_max;
     int keep_res;         // fused stages: also store the stage's residual in res_out (stage 0 of a step)
+    // stage 1 of a global-dt step: the stage state is the update of q0 by tmp, the deferred stage 0
+    // (Stage0Update's operations), formed where it is loaded instead of by a kernel of its own: that
+    // kernel's launch is 2.5 - 4 us of a 25 us step on a 128^2 grid, its 104 bytes a cell 78 of 780 us on
+    // a 2048^2 one.  Variants of their own: in one kernel with the plain load the update's registers cost
+    // the other stages 1 - 9 %.
+    // (the tiles' FOLD variants; the kernel takes the step's dt from the max slots itself)
+    double beta_in, dt_in;   // stage 0's beta and the step's dt
+    int fold_in;             // host execution only, which has no variants
     long long N;
     double cfl;
     const double* q_in;   // stage state [nv][N]
@@ -182,16 +190,36 @@ HC_HD int xcd_tile(int b, int ntiles)
     return start + y;
 }
 
+// q1 = S( C(q0) + R_tot*fac )   (spatial/eulerForwardUpdate.h:76-85), and its status bits
+template <int LAW, int BASIS>
+HC_HD void updated(const Species<double>& sp, const double* q0, const double* Rt, double fac, double* q1, unsigned int& flag)
+{
+    constexpr int NV = LawTraits<LAW>::nv;
+    double qc[NV];
+    to_conserved<double, LAW, BASIS>(sp, q0, qc);
+    for (int v = 0; v < NV; ++v) qc[v] = qc[v] + Rt[v] * fac;
+    from_conserved<double, LAW, BASIS>(sp, qc, q1);
+    bool fin = true;
+    for (int v = 0; v < NV; ++v) fin = fin && hc_isfinite(q1[v]);
+    if (!fin) flag |= ST_NONFINITE;
+    if constexpr (LAW == LAW_EULER && BASIS == BASIS_PRIMITIVE) {
+        if (!(q1[2] > 0.0) || !(q1[3] > 0.0)) flag |= ST_NONPHYSICAL;
+    } else if constexpr (LAW == LAW_EULER) {
+        if (!(q1[2] > 0.0)) flag |= ST_NONPHYSICAL;
+    }
+}
+
 // NTHR threads per work-group, at least one per cell: the extra lanes share the load, metric and
 // face phases, so more waves are resident per SIMD for the same LDS tile.
 // UNI: uniform geometry (a periodic box whose face slots and cell volumes are all equal, checked
 // bitwise on the host): every face takes the slots of face 0 of its kind and every cell the volume
 // of cell 0, read at wave-uniform addresses (scalar loads) instead of one load per face and slot.
 template <int LAW, int BASIS, int FLUX, class RF, int TI, int TJ, int NTHR = TI * TJ, int CST = 0, int GPF = 0,
-          int UNI = 0>
+          int UNI = 0, int FOLD = 0>
 struct StageTile {
     static constexpr int NV = LawTraits<LAW>::nv;
     static constexpr int TILE_I = TI, TILE_J = TJ;
+    static constexpr bool FOLDS = FOLD != 0;
     static constexpr int NC = TI * TJ;   // cells of the tile
     static constexpr int NT = NTHR;      // threads of the work-group
     static_assert(NT >= NC, "one thread per cell at least");
@@ -236,8 +264,17 @@ struct StageTile {
         return g < 0 ? 0 : (g >= n ? n - 1 : g);
     }
 
+    HC_HD static bool folded(const StageArgs<RF>& a)
+    {
+#if defined(__HIP_DEVICE_COMPILE__)
+        return FOLDS;
+#else
+        return a.fold_in != 0;
+#endif
+    }
+
     // ---- phase 1: solution tile with a 2-cell halo ----
-    HC_HD static void load(const StageArgs<RF>& a, Smem& s, int i0, int j0, int tid)
+    HC_HD static void load(const StageArgs<RF>& a, Smem& s, int i0, int j0, int tid, unsigned int& flag)
     {
         const int ni = a.m.ni, nj = a.m.nj;
         for (int k = tid; k < QH * QW; k += NT) {
@@ -245,7 +282,17 @@ struct StageTile {
             const int gi = wrapi(i0 - 2 + li, ni, a.m.per_i);
             const int gj = wrapi(j0 - 2 + lj, nj, a.m.per_j);
             const long long c = (long long)gi * nj + gj;
-            for (int v = 0; v < NV; ++v) s.q[v][li][lj] = QT(a.q_in[v * a.N + c]);
+            if (folded(a)) {
+                double q0[NV], Rt[NV], q1[NV];
+                for (int v = 0; v < NV; ++v) {
+                    q0[v] = a.q0[v * a.N + c];
+                    Rt[v] = a.tmp[v * a.N + c];
+                }
+                updated<LAW, BASIS>(a.sp, q0, Rt, hc_div(a.beta_in * a.dt_in, a.m.cvol[UNI ? 0 : c]), q1, flag);
+                for (int v = 0; v < NV; ++v) s.q[v][li][lj] = QT(q1[v]);
+            } else {
+                for (int v = 0; v < NV; ++v) s.q[v][li][lj] = QT(a.q_in[v * a.N + c]);
+            }
             if constexpr (CSTAGE) {
                 s.gc[0][li][lj] = a.m.ccx[c];
                 s.gc[1][li][lj] = a.m.ccy[c];
@@ -734,7 +781,7 @@ struct StageTile {
         }
         double fac;
         if (a.dt_mode == 0) {
-            const double dt = a.dtslot[0];
+            const double dt = folded(a) ? a.dt_in : a.dtslot[0];
             fac = (p.beta * dt) / vol;
         } else if (a.dt_mode == 2) {
             fac = (p.beta * a.cfl) / vol;   // fixed step: cfl holds dt
@@ -753,25 +800,12 @@ struct StageTile {
         update_cell(a, c, q0, Rt, fac, flag);
     }
 
-    // q_out = S( C(q0) + R_tot*fac )   (spatial/eulerForwardUpdate.h:76-85)
     HC_HD static void update_cell(const StageArgs<RF>& a, long long c, const double* q0, const double* Rt, double fac,
                                   unsigned int& flag)
     {
-        double qc[NV], qn[NV];
-        to_conserved<double, LAW, BASIS>(a.sp, q0, qc);
-        for (int v = 0; v < NV; ++v) qc[v] = qc[v] + Rt[v] * fac;
-        from_conserved<double, LAW, BASIS>(a.sp, qc, qn);
-        bool fin = true;
-        for (int v = 0; v < NV; ++v) {
-            a.q_out[v * a.N + c] = qn[v];
-            fin = fin && hc_isfinite(qn[v]);
-        }
-        if (!fin) flag |= ST_NONFINITE;
-        if constexpr (LAW == LAW_EULER && BASIS == BASIS_PRIMITIVE) {
-            if (!(qn[2] > 0.0) || !(qn[3] > 0.0)) flag |= ST_NONPHYSICAL;
-        } else if constexpr (LAW == LAW_EULER) {
-            if (!(qn[2] > 0.0)) flag |= ST_NONPHYSICAL;
-        }
+        double qn[NV];
+        updated<LAW, BASIS>(a.sp, q0, Rt, fac, qn, flag);
+        for (int v = 0; v < NV; ++v) a.q_out[v * a.N + c] = qn[v];
     }
 };
 
@@ -836,6 +870,8 @@ template <class RF> struct LaunchArgs {
     int vscale, pscale, limiter;
     int mode, dt_mode, stage, reset_max;
     int keep_res;         // fused stages: also store the stage's residual in res_out (stage 0 of a step)
+    int upd_in;           // the launch runs the FOLD variant
+    double beta_in;
     double cfl;
     RkPlan plan;
     const double* q_in;   // packed [nv][N_c] blocks
@@ -867,6 +903,9 @@ template <class RF, int NV> HC_HD StageArgs<RF> case_args(const LaunchArgs<RF>& 
     a.stage = L.stage;
     a.reset_max = L.reset_max;
     a.keep_res = L.keep_res;
+    a.beta_in = L.beta_in;
+    a.dt_in = 0.0;
+    a.fold_in = 0;
     a.N = c.N;
     a.cfl = L.cfl;
     a.q_in = L.q_in + NV * c.cell_off;
@@ -913,6 +952,16 @@ __device__ inline unsigned long long wave_max_u64(unsigned long long v)
 }
 static_assert(MAXSPREAD == 64, "one slot per lane of a wavefront");
 
+// dt = cfl / max(lambda/vol) over a case's slots (rungeKutta.h:133), the same on every lane: one slot per
+// lane, then the wavefront's max (every lane active)
+__device__ inline double step_dt(double cfl, const unsigned long long* maxslot)
+{
+    const unsigned long long m = wave_max_u64(maxslot[(threadIdx.x & 63) * MAXSTRIDE]);
+    const unsigned int lo = __builtin_amdgcn_readfirstlane((unsigned int)m);
+    const unsigned int hi = __builtin_amdgcn_readfirstlane((unsigned int)(m >> 32));
+    return cfl / bits_dbl(((unsigned long long)hi << 32) | lo);
+}
+
 // optional occupancy hint (waves per SIMD) for the register allocator, set per build
 #if defined(HC_STAGE_WAVES_PER_EU) && HC_STAGE_WAVES_PER_EU > 0
 #define HC_STAGE_OCCUPANCY __attribute__((amdgpu_waves_per_eu(HC_STAGE_WAVES_PER_EU)))
@@ -933,6 +982,10 @@ __global__ void __launch_bounds__(T::NT) HC_STAGE_OCCUPANCY __attribute__((amdgp
     const TileRef tr = L.tiles[L.tile_base + xcd_tile(blockIdx.x, L.ntiles)];
     const int ci = tr.ci, lt = tr.lt, i0 = tr.i0, j0 = tr.j0;
     const CaseRec<RF>& c = L.cases[ci];
+    // a folded stage-0 update takes the step's dt from the case's max slots itself, on every wavefront
+    double dt_in = 0.0;
+    if constexpr (T::FOLDS)
+        dt_in = step_dt(L.cfl, L.maxslot + (long long)ci * MAXSPREAD * MAXSTRIDE);
     // The case's parameters (18 array pointers, species, Runge-Kutta plan) held from the first
     // phase to the last exceed the scalar register file, and the kernels then spill them into
     // vector-register lanes (about 110 lane moves per wavefront).  Instead, a group of phases reads
@@ -943,14 +996,18 @@ __global__ void __launch_bounds__(T::NT) HC_STAGE_OCCUPANCY __attribute__((amdgp
     // phase only (a read for their face phase costs them vector registers and time).
     auto args = [&](bool reread = T::REREAD) -> StageArgs<RF> {
         if (!reread) {
-            return case_args<RF, T::NV>(L, c, ci);
+            StageArgs<RF> a = case_args<RF, T::NV>(L, c, ci);
+            a.dt_in = dt_in;
+            return a;
         } else {
             using ConstRec = const __attribute__((address_space(4))) CaseRec<RF>;
             using ConstArgs = const __attribute__((address_space(4))) LaunchArgs<RF>;
             ConstRec* cr = (ConstRec*)&L.cases[__builtin_amdgcn_readfirstlane(ci)];
             ConstArgs* la = (ConstArgs*)__builtin_amdgcn_kernarg_segment_ptr();   // L: the only argument, at offset 0
             asm volatile("" : "+s"(cr), "+s"(la) : : "memory");
-            return case_args<RF, T::NV>(*(const LaunchArgs<RF>*)la, *(const CaseRec<RF>*)cr, ci);
+            StageArgs<RF> a = case_args<RF, T::NV>(*(const LaunchArgs<RF>*)la, *(const CaseRec<RF>*)cr, ci);
+            a.dt_in = dt_in;
+            return a;
         }
     };
     unsigned int flag = 0;
@@ -958,7 +1015,7 @@ __global__ void __launch_bounds__(T::NT) HC_STAGE_OCCUPANCY __attribute__((amdgp
     typename T::CellIn cin;
     {
         const StageArgs<RF> a = args();
-        T::load(a, s, i0, j0, tid);
+        T::load(a, s, i0, j0, tid, flag);
         T::prefetch(a, i0, j0, tid, g0);
         __syncthreads();
         T::qmetric(a, s, i0, j0, tid);
@@ -1004,6 +1061,11 @@ __global__ void __launch_bounds__(T::NT) HC_STAGE_OCCUPANCY __attribute__((amdgp
     }
     // the last stage re-arms the case's max slots for the next step (no stage reads them then)
     if (a.reset_max && lt == 0 && tid < MAXSPREAD) a.maxslot[tid * MAXSTRIDE] = dbl_bits(DBL_MIN);
+    // the later stages read the step's dt, and the case's time advances
+    if (T::FOLDS && lt == 0 && tid == 0) {
+        a.dtslot[0] = dt_in;
+        a.dtslot[1] = a.dtslot[1] + dt_in;
+    }
     // fixed step: the case's time advances once per step (one thread of the case's first tile)
     if (a.dt_mode == 2 && a.mode == MODE_FUSED && a.stage == 0 && lt == 0 && tid == 0) {
         a.dtslot[0] = a.cfl;

@@ -82,6 +82,8 @@ template <class RF> StageArgs<RF> args_of(Emu& e)
 
 // uniform-geometry kernels (UNI) when the case allows them, selected with emu_set_uniform_geometry
 int g_uniform = 0;
+// stage-0 update folded into stage 1's loads
+int g_fold = 0;
 
 template <class T, class RF> void run_tiles(const StageArgs<RF>& a)
 {
@@ -97,7 +99,7 @@ template <class T, class RF> void run_tiles(const StageArgs<RF>& a)
         for (auto& f : flag) f = 0;
         std::vector<typename T::Geo> g0(T::NT);
         for (int tid = 0; tid < T::NT; ++tid) {
-            T::load(a, s, i0, j0, tid);
+            T::load(a, s, i0, j0, tid, flag[tid]);
             T::prefetch(a, i0, j0, tid, g0[tid]);
         }
         for (int tid = 0; tid < T::NT; ++tid) T::qmetric(a, s, i0, j0, tid);
@@ -133,7 +135,7 @@ template <int BASIS, int FLUX, int K> void run_fused_flux(const StageArgs<double
 {
     constexpr TileShape S = TILESF[K];
     if (g_uniform && g_case_uniform) run_tiles<FusedTile<BASIS, FLUX, S.ti, S.tj, S.nt, unsigned, 1>>(a);
-    else if (g_fused == 2) run_tiles<FusedTile<BASIS, FLUX, S.ti, S.tj, S.nt, unsigned long long, 0>>(a);
+    else if (g_fused == 2 && K == 0) run_tiles<FusedTile<BASIS, FLUX, TILESF[0].ti, TILESF[0].tj, TILESF[0].nt, unsigned long long, 0>>(a);
     else run_tiles<FusedTile<BASIS, FLUX, S.ti, S.tj, S.nt, unsigned, 0>>(a);
 }
 
@@ -277,6 +279,13 @@ int emu_set_tile_config(int cfg)
     return 0;
 }
 
+// 1: stage 1 of a global step forms the stage-0 update while it loads (the GPU's sequence); 0: Stage0Update
+int emu_set_fold(int on)
+{
+    g_fold = on;
+    return 0;
+}
+
 // 0: the stage tiles in the reference's order; 1 / 2: the fused Euler tile with 32- / 64-bit offsets
 int emu_set_fused(int mode)
 {
@@ -327,8 +336,16 @@ int emu_integrate(const hc_case_desc* cs, int ni, int nj, const double* nodes, d
             a64.plan = a32.plan = e.plans[s];
             a64.reset_max = a32.reset_max = (global && ns >= 2 && s == ns - 1) ? 1 : 0;
             a64.mode = a32.mode = (global && s == 0) ? MODE_GLOBAL_STAGE0 : MODE_FUSED;
+            const bool fold = g_fold && global && ns >= 3;
+            a64.fold_in = a32.fold_in = fold && s == 1 ? 1 : 0;
+            a64.beta_in = a32.beta_in = e.plans[0].beta;
+            if (a64.fold_in) a64.dt_in = a32.dt_in = cs->cfl / bits_dbl(e.maxslot);
             stage(e, a64, a32);
-            if (global && s == 0) update(e, a64, a32);
+            if (global && s == 0 && !fold) update(e, a64, a32);
+            if (a64.fold_in) {
+                e.dtslot[0] = a64.dt_in;
+                e.dtslot[1] = e.dtslot[1] + a64.dt_in;
+            }
             in = out;
         }
         if (global && ns == 1) e.maxslot = dbl_bits(DBL_MIN);

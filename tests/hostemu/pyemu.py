@@ -54,6 +54,11 @@ def set_fused(mode):
     assert lib().emu_set_fused(int(mode)) == 0
 
 
+def set_fold(on):
+    """1: global-dt steps of three and more stages fold the stage-0 update into stage 1's loads."""
+    lib().emu_set_fold(int(on))
+
+
 def _p(a):
     return a.ctypes.data_as(C.c_void_p)
 
