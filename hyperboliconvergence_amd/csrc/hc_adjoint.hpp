@@ -50,7 +50,7 @@ HC_HD void rk_deliver(const RkDeliver& t, long long i, double x, double vol)
 {
     t.lam[i] = t.lam_add ? t.lam[i] + x : x;
     for (int k = 0; k < t.nk; ++k) {
-        const double y = (t.coef[k] / vol) * x;
+        const double y = hc_div(t.coef[k], vol) * x;
         t.yb[k][i] = t.add[k] ? t.yb[k][i] + y : y;
     }
 }

@@ -163,6 +163,30 @@ __global__ void __launch_bounds__(256) k_soa_to_aos(const double* __restrict__ s
         for (int v = 0; v < nv; ++v) aos[c * nv + v] = soa[v * N + c];
 }
 
+// The slots derived from a direction's FP64 face slots f [NSLOT][nf]: their FP32 copies with the biased LSQ
+// factors replaced by directional weights (fp32_slots' operations), and for a fused context the weights in
+// FP64 as four more planes (directional_weights).  On the host this pass and the upload of the copies
+// were a fifth of setting a case up.
+__global__ void __launch_bounds__(256) k_derive_slots(double* __restrict__ f, float* __restrict__ f32, long long nf, int fused)
+{
+    for (long long k = (long long)blockIdx.x * 256 + threadIdx.x; k < nf; k += (long long)gridDim.x * 256) {
+        for (int s = 0; s < FS_FL0; ++s) f32[s * nf + k] = (float)f[s * nf + k];
+        const double n0 = f[FS_N0 * nf + k], n1 = f[FS_N1 * nf + k];
+        for (int side = 0; side < 2; ++side) {
+            const int s0 = side == 0 ? FS_FL0 : FS_FR0;
+            const double x0 = f[s0 * nf + k], x1 = f[(s0 + 1) * nf + k], x2 = f[(s0 + 2) * nf + k];
+            const double w0 = x0 * n0 + x1 * n1, w1 = x1 * n0 + x2 * n1;
+            f32[s0 * nf + k] = (float)w0;
+            f32[(s0 + 1) * nf + k] = (float)w1;
+            f32[(s0 + 2) * nf + k] = 0.0f;
+            if (fused) {
+                f[(FS_XL0 + 2 * side) * nf + k] = w0;
+                f[(FS_XL1 + 2 * side) * nf + k] = w1;
+            }
+        }
+    }
+}
+
 template <class T> void free_dev(T*& p)
 {
     if (p) (void)hipFree(p);
@@ -430,6 +454,12 @@ int build_tiles(hc_context* ctx)
     return HC_OK;
 }
 
+void derive_slots(hc_context* ctx, double* f, float* f32, long long nf)
+{
+    const unsigned grid = (unsigned)std::min<long long>((nf + 255) / 256, 8192);
+    hipLaunchKernelGGL(k_derive_slots, dim3(grid), dim3(256), 0, ctx->stream, f, f32, nf, ctx->fused ? 1 : 0);
+}
+
 // device layout of all cases: packed arrays, case records, tile tables, update chunks
 int build_layout(hc_context* ctx)
 {
@@ -500,25 +530,15 @@ int build_layout(hc_context* ctx)
             double* fj = ctx->fj + nslot * c.geo_fj_off;
             HC_HIP(hipMemcpy(fi, c.g.fi.data(), c.g.fi.size() * sizeof(double), hipMemcpyHostToDevice));
             HC_HIP(hipMemcpy(fj, c.g.fj.data(), c.g.fj.size() * sizeof(double), hipMemcpyHostToDevice));
-            if (ctx->fused) {
-                std::vector<double> w;
-                directional_weights(c.g.fi, c.nfi, w);
-                HC_HIP(hipMemcpy(fi + NSLOT * c.nfi, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice));
-                directional_weights(c.g.fj, c.nfj, w);
-                HC_HIP(hipMemcpy(fj + NSLOT * c.nfj, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice));
-            }
-            std::vector<float> f32;
-            fp32_slots(c.g.fi, c.nfi, f32);
-            HC_HIP(hipMemcpy(ctx->fi32 + NSLOT * c.geo_fi_off, f32.data(), f32.size() * sizeof(float),
-                             hipMemcpyHostToDevice));
-            fp32_slots(c.g.fj, c.nfj, f32);
-            HC_HIP(hipMemcpy(ctx->fj32 + NSLOT * c.geo_fj_off, f32.data(), f32.size() * sizeof(float),
-                             hipMemcpyHostToDevice));
+            derive_slots(ctx, fi, ctx->fi32 + NSLOT * c.geo_fi_off, c.nfi);
+            derive_slots(ctx, fj, ctx->fj32 + NSLOT * c.geo_fj_off, c.nfj);
+            HC_HIP(hipGetLastError());
         }
         const GeomInput gin{c.ni, c.nj, nullptr, {c.cs.bc[0], c.cs.bc[1], c.cs.bc[2], c.cs.bc[3]}, {0.0, 0.0}, {0.0, 0.0}};
         c.uniform = uniform_geometry(gin, c.g);
         c.X = std::move(c.g.X);
     }
+    HC_HIP(hipStreamSynchronize(ctx->stream));   // the derived slots are written
     for (auto& c : ctx->cases) c.g = GeomOutput{};   // the device holds it now
     // state, accumulators, per-case slots
     for (auto& b : ctx->q) {

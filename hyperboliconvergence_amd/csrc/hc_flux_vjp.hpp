@@ -34,7 +34,7 @@ HC_HD void euler_state_vjp(const Species<double>& sp, double inv_Rg, const doubl
     const double kb = hb;
     const double tb = a2b * (gam * Rg);
     const double v2b = 0.5 * kb;
-    const double inv_r = 1.0 / s.r;
+    const double inv_r = hc_div(1.0, s.r);
     // t = p / (r Rg): dt = dp / (r Rg) - t dr / r
     pb = pb + tb * inv_r * inv_Rg;
     rb = rb - tb * s.t * inv_r;
@@ -71,6 +71,10 @@ HC_HD double ms_m4_d(int sign, double M, double beta)
 }
 HC_HD double ms_p1_d(int sign, double M)
 {
+#if defined(__HIP_DEVICE_COMPILE__)
+    (void)sign;
+    return 0.0 * M;   // P1 is 1 for every |M| below 2^970 (hc_point.hpp ms_p1): the quotient rule leaves some 1e-308
+#endif
     const double eps = NumLimits<double>::max();
     const double inv_b = 1.0 / (hc_fabs(M) + eps);
     const double r = (ms_m1(sign, M) + eps) * inv_b;
@@ -96,8 +100,8 @@ HC_HD double limit_d(int lim, double a, double b, double& da, double& db)
         const double eps = NumLimits<double>::min();
         const double num = b * (a * a) + a * (b * b);
         const double den = a * a + b * b + eps;
-        const double f = num / den;
-        const double inv = 1.0 / den;
+        const double f = hc_div(num, den);
+        const double inv = hc_div(1.0, den);
         da = (2.0 * a * b + b * b - f * (2.0 * a)) * inv;
         db = (a * a + 2.0 * a * b - f * (2.0 * b)) * inv;
         return f;
@@ -121,7 +125,7 @@ HC_HD double ausmpup_vjp(const Species<double>& sp, int vscale, int pscale, cons
     const EState<double> sr = euler_state<double, BASIS>(sp, qr);
     // ---- forward: the intermediates of euler_ausmpup ----
     const double alpha0 = 0.1875, beta = 0.125, Ku = 0.75 * 2.0, Kp = 0.25, sigma = 1.0;
-    const double ascoeff = 2. * (sp.gamma - 1.) / (sp.gamma + 1.);
+    const double ascoeff = hc_div(2. * (sp.gamma - 1.), sp.gamma + 1.);
     const double unl = proj_vel(f.n0, f.n1, sl.u, sl.v);
     const double unr = proj_vel(f.n0, f.n1, sr.u, sr.v);
     const double als2 = ascoeff * sl.h;
@@ -129,16 +133,16 @@ HC_HD double ausmpup_vjp(const Species<double>& sp, int vscale, int pscale, cons
     const double sqal = hc_sqrt(als2), sqar = hc_sqrt(ars2);
     const double dal = hc_fmax(unl, sqal), dar = hc_fmax(-unr, sqar);
     const bool dal_u = dal == unl, dar_u = dar == -unr;
-    const double als = als2 / dal;
-    const double ars = ars2 / dar;
+    const double als = hc_div(als2, dal);
+    const double ars = hc_div(ars2, dar);
     const double ra = 0.5 * (sl.r + sr.r);
     const double as = hc_fmin(ars, als);
     const bool as_r = as == ars;
-    const double ml = unl / as;
-    const double mr = unr / as;
+    const double ml = hc_div(unl, as);
+    const double mr = hc_div(unr, as);
     const double minf = sp.minf;
     const double m0 = hc_sqrt(0.5 * (ml * ml + mr * mr));
-    const double mu = sp.lref / (as * sp.dt);
+    const double mu = hc_div(sp.lref, as * sp.dt);
     // clamp(x, minf, 1): 0 = x, 1 = minf, 2 = 1
     auto clamp_branch = [&](double x) { return x < minf ? 1 : (1.0 < x ? 2 : 0); };
     const int bc = clamp_branch(m0);
@@ -162,7 +166,7 @@ HC_HD double ausmpup_vjp(const Species<double>& sp, int vscale, int pscale, cons
     const double mpc = hc_fmax(mpc0, 0.);
     const bool mpc_x = mpc == mpc0;
     const double D = fa_p * ra * as * as;
-    const double mp = Kp * mpc * delp / D;
+    const double mp = hc_div(Kp * mpc * delp, D);
     const double S = mlp + mrm - mp;
     const double ua = as * S * f.area;
     const double alpha = alpha0 * (5. * fa_u * fa_u - 4.);
@@ -175,7 +179,7 @@ HC_HD double ausmpup_vjp(const Species<double>& sp, int vscale, int pscale, cons
     const double rup = m1l * sl.r + m1r * sr.r;
     const double mdot = ua * rup;
     // ---- reverse ----
-    const double inv_as = 1.0 / as;
+    const double inv_as = hc_div(1.0, as);
     // F0 = mdot u_up + pa n0, F1 = mdot v_up + pa n1, F2 = mdot, F3 = mdot h_up
     const double mdotb = w[0] * (m1l * sl.u + m1r * sr.u) + w[1] * (m1l * sl.v + m1r * sr.v) + w[2] +
                          w[3] * (m1l * sl.h + m1r * sr.h);
@@ -221,7 +225,7 @@ HC_HD double ausmpup_vjp(const Species<double>& sp, int vscale, int pscale, cons
     mrb += Sb * (mrsub * ms_m4_d(-1, mr, beta) + mrsup * ms_m1_d(-1, mr));
     const double mpb = -Sb;
     // mp = Kp mpc delp / D, D = fa_p ra as as
-    const double inv_D = 1.0 / D;
+    const double inv_D = hc_div(1.0, D);
     const double mpcb = mpb * Kp * delp * inv_D;
     const double delpb = mpb * Kp * mpc * inv_D;
     const double Db = -mpb * mp * inv_D;
@@ -248,7 +252,7 @@ HC_HD double ausmpup_vjp(const Species<double>& sp, int vscale, int pscale, cons
         else asb += m0_ab * (-mu * inv_as);   // mu = lref / (as dt)
     }
     // m0 = sqrt(0.5 (ml^2 + mr^2))
-    const double Y = m0b * (0.5 / m0);
+    const double Y = m0b * hc_div(0.5, m0);
     mlb += Y * ml;
     mrb += Y * mr;
     // ml = unl / as, mr = unr / as
@@ -261,16 +265,16 @@ HC_HD double ausmpup_vjp(const Species<double>& sp, int vscale, int pscale, cons
     rlb += 0.5 * rab;
     rrb += 0.5 * rab;
     // als = als2 / fmax(unl, sqrt(als2)), ars = ars2 / fmax(-unr, sqrt(ars2))
-    const double inv_dal = 1.0 / dal;
+    const double inv_dal = hc_div(1.0, dal);
     double als2b = alsb * inv_dal;
     const double dalb = -alsb * als * inv_dal;
     if (dal_u) unlb += dalb;
-    else als2b += dalb * (0.5 / sqal);
-    const double inv_dar = 1.0 / dar;
+    else als2b += dalb * hc_div(0.5, sqal);
+    const double inv_dar = hc_div(1.0, dar);
     double ars2b = arsb * inv_dar;
     const double darb = -arsb * ars * inv_dar;
     if (dar_u) unrb -= darb;
-    else ars2b += darb * (0.5 / sqar);
+    else ars2b += darb * hc_div(0.5, sqar);
     hlb += als2b * ascoeff;
     hrb += ars2b * ascoeff;
     // un = n0 u + n1 v
@@ -278,7 +282,7 @@ HC_HD double ausmpup_vjp(const Species<double>& sp, int vscale, int pscale, cons
     vlb += unlb * f.n1;
     urb += unrb * f.n0;
     vrb += unrb * f.n1;
-    const double inv_Rg = 1.0 / sp.Rg;
+    const double inv_Rg = hc_div(1.0, sp.Rg);
     euler_state_vjp<BASIS>(sp, inv_Rg, ql, sl, ulb, vlb, rlb, plb, hlb, 0.0, qlb);
     euler_state_vjp<BASIS>(sp, inv_Rg, qr, sr, urb, vrb, rrb, prb, hrb, 0.0, qrb);
     return minfb;
