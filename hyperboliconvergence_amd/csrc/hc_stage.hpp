@@ -326,6 +326,10 @@ struct StageTile {
         const RF* fi = a.m.fi;
         const RF* fj = a.m.fj;
         const long long nfi = a.m.nfi, nfj = a.m.nfj;
+        // A tile whose ring has all its neighbours inside the mesh (the same on every lane) takes its four
+        // edges without the per-lane side tests, in the same order: 100 instructions a ring cell for 190 (48 mixed
+        // cylinders 7223 -> 7115 us for 10 steps, the ordered FP64 kernels 1.2 %).
+        const bool inner = i0 >= 2 && i0 + TI + 1 < ni && j0 >= 2 && j0 + TJ + 1 < nj;
         for (int k = tid; k < MH * MW; k += NT) {
             const int li = k / MW, lj = k % MW;
             const int ri = i0 - 1 + li, rj = j0 - 1 + lj;   // unwrapped global index
@@ -359,6 +363,14 @@ struct StageTile {
                     acc[v][1] = acc[v][1] + dq * dx1;
                 }
             };
+            if (inner) {
+                edge(r - 1, c, r, c, fi, nfi, (long long)gi * nj + gj, false);
+                edge(r, c, r + 1, c, fi, nfi, (long long)(gi + 1) * nj + gj, false);
+                edge(r, c - 1, r, c, fj, nfj, (long long)gi * (nj + 1) + gj, false);
+                edge(r, c, r, c + 1, fj, nfj, (long long)gi * (nj + 1) + gj + 1, false);
+                put_metric(s, li, lj, acc);
+                continue;
+            }
             if (gi > 0) edge(r - 1, c, r, c, fi, nfi, (long long)gi * nj + gj, false);
             if (gi < ni - 1) edge(r, c, r + 1, c, fi, nfi, (long long)(gi + 1) * nj + gj, false);
             if (gj > 0) edge(r, c - 1, r, c, fj, nfj, (long long)gi * (nj + 1) + gj, false);
@@ -371,10 +383,15 @@ struct StageTile {
                 if (gj == 0) edge(r, c - 1, r, c, fj, nfj, (long long)gi * (nj + 1), true);
                 if (gj == nj - 1) edge(r, c, r, c + 1, fj, nfj, (long long)gi * (nj + 1), true);
             }
-            for (int v = 0; v < NV; ++v) {
-                s.Q[v][0][li][lj] = acc[v][0];
-                s.Q[v][1][li][lj] = acc[v][1];
-            }
+            put_metric(s, li, lj, acc);
+        }
+    }
+
+    HC_HD static void put_metric(Smem& s, int li, int lj, const RF (*acc)[2])
+    {
+        for (int v = 0; v < NV; ++v) {
+            s.Q[v][0][li][lj] = acc[v][0];
+            s.Q[v][1][li][lj] = acc[v][1];
         }
     }
 

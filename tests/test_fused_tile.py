@@ -117,3 +117,19 @@ def test_folded_stage0_update_gives_the_update_kernels_bits(rk, mode, precision)
         pyemu.set_fold(0)
         assert out[0][2] == out[1][2] == 0
         assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("flux", [po.FLUX_ROE_FACEFRAME, po.FLUX_SLAU])
+def test_ordered_tiles_inside_the_mesh(flux, precision):
+    """Tiles away from every side take their metric without the side tests, in the same order: the oracle's
+    bits in FP64, and in both precisions the bits of shapes whose tiles lie elsewhere."""
+    cs, nodes, q, bref = _ogrid(26, 70, 1, flux, po.LIM_MINMOD2)
+    pyemu.set_fused(0)
+    out = []
+    for shape in range(3):
+        pyemu.set_tile_config(shape)
+        out.append(pyemu.residual(cs, nodes, q, bref, precision)[0])
+        assert np.array_equal(out[-1], out[0])
+    if precision == 0:
+        assert np.array_equal(out[0], po.residual(cs, nodes, q, bref))
