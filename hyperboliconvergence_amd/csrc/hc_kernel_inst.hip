@@ -44,9 +44,14 @@ template <int K, int UNI, class A> static hipError_t launch_shape(const A& L, hi
     // centre staging has nothing to stage on uniform geometry, so a shape that differs from another
     // only by it shares that shape's kernel
     constexpr hc::TileShape S = hc::tile_shapes(HC_PREC == 32, HC_LAW, HC_FLUX, false)[K];
-    constexpr int WPE = S.gpf != 0 ? 4 : 1, CST = UNI ? 0 : S.cst;
+    // FP64 in the reference's order takes 91 - 97 VGPRs where the cell phase's inputs are loaded late: five
+    // waves per SIMD ask for 96 (AUSM+up in the primitive basis holds them early, at four): the 512x1024
+    // gradient 5190 -> 5104 us; the variants that fold an update would spill there and keep four
+    constexpr int CST = UNI ? 0 : S.cst;
+    constexpr bool EARLY = HC_LAW == 1 && HC_FLUX == 4 && HC_BASIS == 1;
+    constexpr int WPE = S.gpf == 0 ? 1 : HC_PREC == 64 && HC_LAW == 1 && !EARLY && !UNI ? 5 : 4;
     if (L.upd_in)
-        return launch<hc::StageTile<HC_LAW, HC_BASIS, HC_FLUX, RF, S.ti, S.tj, S.nt, CST, S.gpf, UNI, 1>, WPE>(L, st);
+        return launch<hc::StageTile<HC_LAW, HC_BASIS, HC_FLUX, RF, S.ti, S.tj, S.nt, CST, S.gpf, UNI, 1>, (S.gpf != 0 ? 4 : 1)>(L, st);
     return launch<hc::StageTile<HC_LAW, HC_BASIS, HC_FLUX, RF, S.ti, S.tj, S.nt, CST, S.gpf, UNI>, WPE>(L, st);
 }
 
