@@ -65,9 +65,9 @@ struct hc_context {
     float *fi32 = nullptr, *fj32 = nullptr;
     double* q[3] = {nullptr, nullptr, nullptr};
     int cur = 0;
-    double *acc = nullptr, *tmp = nullptr, *lam0 = nullptr, *bref = nullptr, *res = nullptr, *part = nullptr,
+    double *acc = nullptr, *tmp = nullptr, *tmp2 = nullptr, *lam0 = nullptr, *bref = nullptr, *res = nullptr, *part = nullptr,
            *nout = nullptr;
-    unsigned long long* maxslot = nullptr;   // MAXSPREAD slots per case, MAXSTRIDE words apart
+    unsigned long long* maxslot = nullptr;   // three sets (enqueue_steps) of MAXSPREAD slots per case, MAXSTRIDE words apart
     double* dtslot = nullptr;                // two per case
     unsigned int* status = nullptr;
     CaseRec<double>* rec64[NTILECFG] = {};

@@ -12,6 +12,14 @@
 // Sums at the sides are in another order than the oracle's and products are fused: results agree to
 // rounding (1e-13 of the residual), and are the same bits in every tile shape, since every fused
 // operation is explicit.
+//
+// Bound: latency of the load phase, then instruction issue (96 cylinders, a wavefront's 15.1k cycles: waits
+// for the record and the tile 5.4k, metric 1.7k, faces 3.8k, cells 1.8k, barriers 2.4k; VALU busy 61 % at
+// 4.2 waves a SIMD).  Against StageTile: the same 96 cylinders 18.9 -> 13.9 ms for 10 steps, a 2048x2048
+// AUSM+up box 7.66 -> 2.99 ms for 4, a 256x512 cylinder 1.44 -> 1.00 ms for 20.
+// Tried and slower: six waves with the fluxes stored over the state tile (spills off uniform geometry: 96
+// cylinders 13.98 -> 15.07 ms), a persistent loop that loads the next tile during the cell phase (2048x2048
+// 3.15 -> 3.76 ms).
 #pragma once
 
 #include "hc_fused_flux.hpp"
@@ -127,11 +135,15 @@ template <int BASIS, int FLUX, int TI, int TJ, int NTHR, class Off, int UNI, int
                 double q0[NV], Rt[NV], q1[NV];
                 for (int v = 0; v < NV; ++v) {
                     q0[v] = at(a.q0 + v * a.N, o);
-                    Rt[v] = at(a.tmp + v * a.N, o);
+                    Rt[v] = at(a.tmp_in + v * a.N, o);
                 }
                 const double vol = UNI ? uniform(a.m.cvol) : at(a.m.cvol, o);
                 advance(a, q0, Rt, hc_div(a.beta_in * a.dt_in, vol), q1, flag);
                 for (int v = 0; v < NV; ++v) s.q[v][li][lj] = q1[v];
+                // a one-stage table: the update is the step's result
+                if (a.mode == MODE_GLOBAL_STAGE0 && li >= 2 && li < TI + 2 && lj >= 2 && lj < TJ + 2 &&
+                    i0 - 2 + li < a.m.ni && j0 - 2 + lj < a.m.nj)
+                    for (int v = 0; v < NV; ++v) put(a.q_out + v * a.N, o, q1[v]);
             } else {
                 for (int v = 0; v < NV; ++v) s.q[v][li][lj] = at(a.q_in + v * a.N, o);
             }

@@ -15,6 +15,9 @@
 //               reference's order (spatial/residualCalc.h:199-305), no atomics,
 //               then the Runge-Kutta accumulation and forward-Euler update
 //               (timestepping/rungeKutta.h:176-197, spatial/eulerForwardUpdate.h)
+// StageTile keeps the reference's operation order, so FP64 results are the oracle's bits.  It runs the
+// mixed path, scalar advection, the verbatim Roe and SLAU fluxes and fixed-step contexts; the other Euler
+// fluxes run in FP64 as FusedTile (hc_fused.hpp), by fused_euler() in hc_point.hpp.
 // The phases are __host__ __device__ so that a work-group can be executed
 // thread by thread on the host for debugging; the kernel wrappers are at the end.
 #pragma once
@@ -143,6 +146,7 @@ template <class RF> struct StageArgs {
     double* q_out;        // [nv][N]
     double* acc;          // accumulators [slot][nv][N]
     double* tmp;          // deferred R_tot of global-dt stage 0 [nv][N]
+    const double* tmp_in; // the same, as a folded update reads it
     double* lam0;         // stage-0 spectral radius sums [N]
     const double* bref;   // boundary reference values, AoS [2nj+2ni][nv]
     double* res_out;      // residual-only mode: AoS [N][nv+1]
@@ -286,10 +290,14 @@ struct StageTile {
                 double q0[NV], Rt[NV], q1[NV];
                 for (int v = 0; v < NV; ++v) {
                     q0[v] = a.q0[v * a.N + c];
-                    Rt[v] = a.tmp[v * a.N + c];
+                    Rt[v] = a.tmp_in[v * a.N + c];
                 }
                 updated<LAW, BASIS>(a.sp, q0, Rt, hc_div(a.beta_in * a.dt_in, a.m.cvol[UNI ? 0 : c]), q1, flag);
                 for (int v = 0; v < NV; ++v) s.q[v][li][lj] = QT(q1[v]);
+                // a one-stage table: the update is the step's result
+                if (a.mode == MODE_GLOBAL_STAGE0 && li >= 2 && li < TI + 2 && lj >= 2 && lj < TJ + 2 &&
+                    i0 - 2 + li < ni && j0 - 2 + lj < nj)
+                    for (int v = 0; v < NV; ++v) a.q_out[v * a.N + c] = q1[v];
             } else {
                 for (int v = 0; v < NV; ++v) s.q[v][li][lj] = QT(a.q_in[v * a.N + c]);
             }
@@ -902,6 +910,10 @@ template <class RF> struct LaunchArgs {
     unsigned long long* maxslot;   // MAXSPREAD * MAXSTRIDE per case
     double* dtslot;                // two per case
     unsigned int* status;
+    // a folded update: the residuals it reads, the slots it takes its dt from, slots to re-arm (null: none)
+    const double* tmp_in;
+    const unsigned long long* max_in;
+    unsigned long long* max_next;
 };
 
 // the single-case view of case ci of a batched launch
@@ -930,6 +942,7 @@ template <class RF, int NV> HC_HD StageArgs<RF> case_args(const LaunchArgs<RF>& 
     a.q_out = L.q_out + NV * c.cell_off;
     a.acc = L.nslots > 0 ? L.acc + (long long)L.nslots * NV * c.cell_off : nullptr;
     a.tmp = L.tmp + NV * c.cell_off;
+    a.tmp_in = L.tmp_in + NV * c.cell_off;
     a.lam0 = L.lam0 + c.cell_off;
     a.bref = L.bref + NV * c.bref_off;
     a.res_out = L.res_out + (NV + 1) * c.cell_off;
@@ -999,10 +1012,10 @@ __global__ void __launch_bounds__(T::NT) HC_STAGE_OCCUPANCY __attribute__((amdgp
     const TileRef tr = L.tiles[L.tile_base + xcd_tile(blockIdx.x, L.ntiles)];
     const int ci = tr.ci, lt = tr.lt, i0 = tr.i0, j0 = tr.j0;
     const CaseRec<RF>& c = L.cases[ci];
-    // a folded stage-0 update takes the step's dt from the case's max slots itself, on every wavefront
+    // a folded update takes the step's dt from the case's max slots itself, on every wavefront
     double dt_in = 0.0;
     if constexpr (T::FOLDS)
-        dt_in = step_dt(L.cfl, L.maxslot + (long long)ci * MAXSPREAD * MAXSTRIDE);
+        dt_in = step_dt(L.cfl, L.max_in + (long long)ci * MAXSPREAD * MAXSTRIDE);
     // The case's parameters (18 array pointers, species, Runge-Kutta plan) held from the first
     // phase to the last exceed the scalar register file, and the kernels then spill them into
     // vector-register lanes (about 110 lane moves per wavefront).  Instead, a group of phases reads
@@ -1078,6 +1091,8 @@ __global__ void __launch_bounds__(T::NT) HC_STAGE_OCCUPANCY __attribute__((amdgp
     }
     // the last stage re-arms the case's max slots for the next step (no stage reads them then)
     if (a.reset_max && lt == 0 && tid < MAXSPREAD) a.maxslot[tid * MAXSTRIDE] = dbl_bits(DBL_MIN);
+    if (T::FOLDS && L.max_next && lt == 0 && tid < MAXSPREAD)
+        L.max_next[((long long)ci * MAXSPREAD + tid) * MAXSTRIDE] = dbl_bits(DBL_MIN);
     // the later stages read the step's dt, and the case's time advances
     if (T::FOLDS && lt == 0 && tid == 0) {
         a.dtslot[0] = dt_in;

@@ -71,6 +71,7 @@ template <class RF> StageArgs<RF> args_of(Emu& e)
     a.cfl = e.cs.cfl;
     a.acc = e.acc.data();
     a.tmp = e.tmp.data();
+    a.tmp_in = a.tmp;
     a.lam0 = e.lam0.data();
     a.bref = e.bref.data();
     a.res_out = e.res.data();
@@ -320,7 +321,37 @@ int emu_integrate(const hc_case_desc* cs, int ni, int nj, const double* nodes, d
     if (setup(e, cs, ni, nj, nodes, q, bref, precision)) return -1;
     const int ns = cs->nstages;
     const bool global = cs->dt_mode == HC_DT_GLOBAL;
-    for (int step = 0; step < nsteps; ++step) {
+    // one-stage steps chained as hc_capi.cpp enqueue_steps: residual kernels that update as they load, and
+    // one update at the end
+    const bool chain = g_fold && global && ns == 1 && nsteps > 1;
+    std::vector<double> tmp2(chain ? e.tmp.size() : 0);
+    for (int step = 0; chain && step <= nsteps; ++step) {
+        StageArgs<double> a64 = args_of<double>(e);
+        StageArgs<float> a32 = args_of<float>(e);
+        double* tmp[2] = {e.tmp.data(), tmp2.data()};
+        a64.q_in = a32.q_in = a64.q0 = a32.q0 = e.q[e.cur].data();
+        a64.q_out = a32.q_out = e.q[1 - e.cur].data();
+        a64.plan = a32.plan = e.plans[0];
+        a64.beta_in = a32.beta_in = e.plans[0].beta;
+        a64.mode = a32.mode = MODE_GLOBAL_STAGE0;
+        a64.tmp = a32.tmp = tmp[(step == nsteps ? step + 1 : step) % 2];
+        a64.tmp_in = a32.tmp_in = tmp[(step + 1) % 2];
+        if (step == nsteps) {
+            update(e, a64, a32);
+            e.maxslot = dbl_bits(DBL_MIN);
+        } else {
+            a64.fold_in = a32.fold_in = step > 0 ? 1 : 0;
+            if (step > 0) {
+                a64.dt_in = a32.dt_in = cs->cfl / bits_dbl(e.maxslot);
+                e.dtslot[0] = a64.dt_in;
+                e.dtslot[1] = e.dtslot[1] + a64.dt_in;
+            }
+            e.maxslot = dbl_bits(DBL_MIN);
+            stage(e, a64, a32);
+        }
+        if (step > 0) e.cur = 1 - e.cur;
+    }
+    for (int step = 0; !chain && step < nsteps; ++step) {
         double* q0 = e.q[e.cur].data();
         double* bufA = ns == 1 ? e.q[1 - e.cur].data() : e.q[(e.cur + 1) % 3].data();
         double* bufB = ns == 1 ? bufA : e.q[(e.cur + 2) % 3].data();

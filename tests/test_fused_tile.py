@@ -103,10 +103,10 @@ def test_uniform_geometry_gives_the_general_tiles_bits(flux):
         assert np.array_equal(pyemu.integrate(cs, nodes, q, bref, 2)[0], steps[0])
 
 
-@pytest.mark.parametrize("rk", [33, 34, 44])
+@pytest.mark.parametrize("rk", [11, 33, 34, 44])
 @pytest.mark.parametrize("mode", [0, 1], ids=["ordered", "fused"])
 @pytest.mark.parametrize("precision", [0, 1])
-def test_folded_stage0_update_gives_the_update_kernels_bits(rk, mode, precision):
+def test_folded_updates_give_the_update_kernels_bits(rk, mode, precision):
     for flux, box in ((po.FLUX_AUSMPUP, True), (po.FLUX_ROE_FACEFRAME, False)):
         args = _box(5, 21, flux, False) if box else _ogrid(10, 18, 1, flux, po.LIM_MINMOD2, dt=po.DT_GLOBAL, rk=rk)
         out = []
