@@ -243,7 +243,7 @@ def stage_counter(rows, counter, rf, triad_n):
         if row.get("Counter_Name") != counter:
             continue
         per.setdefault(row["Kernel_Name"], []).append(float(row["Counter_Value"]))
-    stage = [(len(v), k) for k, v in per.items() if k.startswith("void hc::k_stage<") and f", {rf}, " in k]
+    stage = [(len(v), k) for k, v in per.items() if k.startswith("void hc::k_stage<") and f"LaunchArgs<{rf}>" in k]
     scale = [v for k, v in per.items() if "k_scale8" in k]
     if not stage or not scale or float(np.mean(scale[0])) <= 0:
         return None

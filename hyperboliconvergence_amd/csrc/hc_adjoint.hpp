@@ -6,7 +6,8 @@
 // boundary reference states (used by the far-field boundary conditions).
 //
 //   tangent:  given (q, qdot, minf_dot, bref_dot), the kernels return R(q) (bit-identical
-//             to the stage kernel's residual: same operations in the same order) and
+//             to the residual of StageTile, which every fixed-step context runs: same
+//             operations in the same order; equal to FusedTile's to rounding) and
 //             Rdot = dR/dq qdot + dR/dminf minf_dot + dR/dbref bref_dot, by evaluating the
 //             point functions of hc_point.hpp on Dual<1> numbers.
 //   adjoint:  given ybar, the kernels return qbar = (dR/dq)^T ybar, minf_bar and bref_bar.

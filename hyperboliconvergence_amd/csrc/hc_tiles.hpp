@@ -12,11 +12,14 @@ struct TileShape {
     int gpf;          // geometry prefetch: each lane's first face slots loaded before the metric phase
 };
 
-// Three configurations per precision; a context times each on its own cases and keeps the
-// fastest (results are bit-identical).  The face phase runs 2*ti*tj + ti + tj faces on nt lanes:
+// Three configurations per kernel family; a context times each on its own cases and keeps the
+// fastest (results are bit-identical).  Configuration 0 runs where a context takes too few steps to
+// time them, so it is the one that is best or close to it everywhere.
+// The face phase runs 2*ti*tj + ti + tj faces on nt lanes:
+//   7x16 on 256 lanes: 247 faces, one per lane, every wave equally loaded; best on most grids (the
+//        2048x2048 vortex, untimed: 574 us a stage with 4x32 first, 505 with 7x16, before FusedTile)
 //   4x32 on 256 lanes: 292 faces (one wave takes two), 128 cells per work-group; at 4
 //        work-groups per CU a 131072-cell grid is exactly one round of work-groups
-//   7x16 on 256 lanes: 247 faces, one per lane, every wave equally loaded
 // Centre staging reads the cell centres of the q tile (16 B per halo cell) instead of two face
 // slots per metric edge and face (about 10 % fewer bytes and load instructions): it pays on
 // large grids, where work-groups of many rounds overlap their phases, and costs on a grid of
@@ -33,7 +36,8 @@ constexpr TileShape TILES64[NTILECFG] = {{7, 16, 256, 1, 1}, {7, 16, 256, 0, 1},
 constexpr TileShape TILES32[NTILECFG] = {{8, 32, 256, 0, 0}, {7, 32, 256, 0, 0}, {7, 16, 256, 0, 0}};
 
 // Euler in FP64 (FusedTile): one face per lane, i-faces in whole wavefronts, centres staged and face
-// slots prefetched in all of them.
+// slots prefetched in all of them.  7x16 first; 7x8 fills the chip on small grids, 15x16 reads fewer
+// halo cells on large ones.  4x32 would give one wave two faces.
 constexpr TileShape TILESF[NTILECFG] = {{7, 16, 256, 1, 1}, {7, 8, 128, 1, 1}, {15, 16, 512, 1, 1}};
 
 constexpr const TileShape* tile_shapes(bool mixed, int law, int flux, bool fused)

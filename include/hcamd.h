@@ -177,7 +177,7 @@ int hc_set_graph_steps(hc_context* ctx, int k);
  * launch (graphs off); mode 2: one event pair around each hc_step call (graphs on), the
  * interval counted against the stage kernels it launched.  hc_get_profile returns the sums
  * {stage kernel ms, stage-kernel launches, update kernel ms, update launches} since the last
- * hc_set_profiling.  Used for the roofline report.
+ * hc_set_profiling (updates that a stage kernel forms while it loads its tiles launch nothing).  Used for the roofline report.
  */
 int hc_set_profiling(hc_context* ctx, int enable);
 int hc_get_profile(hc_context* ctx, double* out4);
@@ -218,8 +218,8 @@ int hc_batch_norms(hc_context* ctx, int case_id, double* l2, double* linf);
 int hc_batch_get_time(hc_context* ctx, int case_id, double* t);
 
 /*
- * Tile configuration of the stage kernels (shape, and whether the centre differences are
- * formed from cell centres in LDS): config -1 (default) times every configuration on the first
+ * Tile configuration of the stage kernels (shape of the tiles, and in some kernels whether the centre
+ * differences are formed from cell centres in LDS): config -1 (default) times every configuration on the first
  * steps of the context (all give bit-identical results) and keeps the fastest; 0 .. 2 fixes one.
  * hc_get_tiles returns the configuration in use and, after timing, the milliseconds per step of
  * each (HC_NTILECFG values).  No counterpart in the reference.
