@@ -164,8 +164,8 @@ __global__ void __launch_bounds__(256) k_soa_to_aos(const double* __restrict__ s
 }
 
 // The slots derived from a direction's FP64 face slots f [NSLOT][nf]: their FP32 copies with the biased LSQ
-// factors replaced by directional weights (fp32_slots' operations), and for a fused context the weights in
-// FP64 as four more planes (directional_weights).  On the host this pass and the upload of the copies
+// factors replaced by directional weights (fp32_slots' operations), and for a fused context their
+// scaled forms in FP64 as five more planes (directional_weights).  On the host this pass and the upload of the copies
 // were a fifth of setting a case up.
 __global__ void __launch_bounds__(256) k_derive_slots(double* __restrict__ f, float* __restrict__ f32, long long nf, int fused)
 {
@@ -180,10 +180,12 @@ __global__ void __launch_bounds__(256) k_derive_slots(double* __restrict__ f, fl
             f32[(s0 + 1) * nf + k] = (float)w1;
             f32[(s0 + 2) * nf + k] = 0.0f;
             if (fused) {
-                f[(FS_XL0 + 2 * side) * nf + k] = w0;
-                f[(FS_XL1 + 2 * side) * nf + k] = w1;
+                const double d = f[(side == 0 ? FS_DL : FS_DR) * nf + k];
+                f[(FS_XL0 + 2 * side) * nf + k] = d * w0;
+                f[(FS_XL1 + 2 * side) * nf + k] = d * w1;
             }
         }
+        if (fused) f[FS_XS * nf + k] = f[FS_DL * nf + k] * f[FS_S1 * nf + k];
     }
 }
 
@@ -470,7 +472,9 @@ int build_layout(hc_context* ctx)
     ctx->nv = ctx->cs.law == HC_LAW_EULER ? 4 : 3;
     // a fixed step is the form that is differentiated (hc_adjoint.cpp): it keeps the reference's order,
     // since the derivative of a limiter at slopes that almost vanish depends on their last bits
-    ctx->fused = fused_euler(ctx->cs.law, ctx->cs.flux) && ctx->cs.dt_mode != HC_DT_FIXED;
+    // van Leer's ratio is not homogeneous in the slopes, which the scaled weights of the fused tile rely on
+    ctx->fused = fused_euler(ctx->cs.law, ctx->cs.flux) && ctx->cs.dt_mode != HC_DT_FIXED &&
+                 ctx->cs.limiter != LIM_VANLEER2;
     ctx->nslots = make_rk_plans(ctx->cs.nstages, ctx->cs.alpha, ctx->cs.beta, ctx->plans);
     const int nv = ctx->nv;
     const int nc = (int)ctx->cases.size();

@@ -5,8 +5,12 @@
 //               non-periodic side the outermost cell again
 //   2. qmetric: Q = sum over the four neighbours of dq (x) dx; a repeated cell adds zero, so every ring
 //               cell takes the same straight-line path
-//   3. faces  : slopes along the normal from the directional weights w = X'^-1 n of the biased LSQ
-//               factors (4 values a face instead of 6, and 4 operations a slope instead of 9)
+//   3. faces  : increments d lim(g_c, g.n) from the directional weights w = X'^-1 n of the biased LSQ
+//               factors (4 values a face instead of 6, and 4 operations a slope instead of 9).  Every
+//               limiter but van Leer's (whose contexts keep StageTile) is homogeneous, d lim(a, b) = lim(d a, d b), so the weights hold the
+//               distance d and the centred increment is the cell's share of the jump: 8 slots a face
+//               for 10 (a 1000x901 AUSM+up box, bound by these bytes, 1376 -> 1242 us for 6 steps;
+//               96 cylinders 13.87 -> 13.59 ms for 10)
 //   4. cells  : R = F_left - F_right of the four faces (the wall flux of the far sides is stored
 //               negated), then the Runge-Kutta accumulation and the update as StageTile has them
 // Sums at the sides are in another order than the oracle's and products are fused: results agree to
@@ -15,7 +19,7 @@
 //
 // Bound: latency of the load phase, then instruction issue (96 cylinders, a wavefront's 15.1k cycles: waits
 // for the record and the tile 5.4k, metric 1.7k, faces 3.8k, cells 1.8k, barriers 2.4k; VALU busy 61 % at
-// 4.2 waves a SIMD).  Against StageTile: the same 96 cylinders 18.9 -> 13.9 ms for 10 steps, a 2048x2048
+// 4.2 waves a SIMD).  Against StageTile: the same 96 cylinders 18.9 -> 13.6 ms for 10 steps, a 2048x2048
 // AUSM+up box 7.66 -> 2.99 ms for 4, a 256x512 cylinder 1.44 -> 1.00 ms for 20.
 // Tried and slower: six waves with the fluxes stored over the state tile (spills off uniform geometry: 96
 // cylinders 13.98 -> 15.07 ms), a persistent loop that loads the next tile during the cell phase (2048x2048
@@ -49,7 +53,7 @@ template <int BASIS, int FLUX, int TI, int TJ, int NTHR, class Off, int UNI, int
         double gc[2][CH][CW];
     };
     struct Geo {
-        double area, n0, n1, dl, dr, s1, wl0, wl1, wr0, wr1;
+        double area, n0, n1, sl, wl0, wl1, wr0, wr1;
     };
     struct CellIn {
         double q0[NV], acc[NV], old[2][NV], vol, lam0;
@@ -213,9 +217,7 @@ template <int BASIS, int FLUX, int TI, int TJ, int NTHR, class Off, int UNI, int
         g.area = slot(b + FS_AREA * nf, o);
         g.n0 = slot(b + FS_N0 * nf, o);
         g.n1 = slot(b + FS_N1 * nf, o);
-        g.dl = slot(b + FS_DL * nf, o);
-        g.dr = slot(b + FS_DR * nf, o);
-        g.s1 = slot(b + FS_S1 * nf, o);
+        g.sl = slot(b + FS_XS * nf, o);
         g.wl0 = slot(b + FS_XL0 * nf, o);
         g.wl1 = slot(b + FS_XL1 * nf, o);
         g.wr0 = slot(b + FS_XR0 * nf, o);
@@ -284,18 +286,19 @@ template <int BASIS, int FLUX, int TI, int TJ, int NTHR, class Off, int UNI, int
                 }
                 const double* Qr = &s.Q[0][0][0][0] + (li + 1) * MW + lj + 1;
                 const double* Ql = Qr - (isi ? MW : 1);
-                double c[NV], gl[NV], gr[NV], sl[NV], sr[NV];
+                double cl[NV], cr[NV], gl[NV], gr[NV], sl[NV], sr[NV];
                 for (int v = 0; v < NV; ++v) {
                     const double dq = qr[v] - ql[v];
                     const int k0 = 2 * v * MH * MW, k1 = k0 + MH * MW;
-                    c[v] = dq * g.s1;
+                    cl[v] = dq * g.sl;
+                    cr[v] = dq - cl[v];
                     gl[v] = hc_fma(hc_fma(-dq, dy, Ql[k1]), g.wl1, hc_fma(-dq, dx, Ql[k0]) * g.wl0);
                     gr[v] = hc_fma(hc_fma(-dq, dy, Qr[k1]), g.wr1, hc_fma(-dq, dx, Qr[k0]) * g.wr0);
                 }
-                fused_limit4(a.limiter, c, gl, gr, sl, sr);
+                fused_limit4(a.limiter, cl, gl, cr, gr, sl, sr);
                 for (int v = 0; v < NV; ++v) {
-                    ql[v] = hc_fma(sl[v], g.dl, ql[v]);
-                    qr[v] = hc_fma(-sr[v], g.dr, qr[v]);
+                    ql[v] = ql[v] + sl[v];
+                    qr[v] = qr[v] - sr[v];
                 }
             }
             fused_flux<BASIS, FLUX>(a.sp, a.vscale, a.pscale, g.area, g.n0, g.n1, wl, ql, qr, F, lam);

@@ -238,42 +238,40 @@ HC_HD void fused_flux(const Species<double>& sp, int vscale, int pscale, double 
     else fused_ausmpup(sp, vscale, pscale, area, n0, n1, wl, L, R, F, lam);
 }
 
-// Limiter L of a centred slope a with the biased slopes bl, br (limiters/limiter.ipp).  van Albada:
+// Limiter L of a centred increment a with a biased one b (limiters/limiter.ipp).  van Albada:
 // b a^2 + a b^2 = ab (a + b), and the switch on a b < 0 is a maximum with zero; MinMod: the biased
-// slope clamped to [min(a, 0), max(a, 0)].
-template <int L> HC_HD void fused_limit(double a, double bl, double br, double& sl, double& sr)
+// increment clamped to [min(a, 0), max(a, 0)].
+template <int L> HC_HD double fused_limit(double a, double b)
 {
     if constexpr (L == LIM_VANALBADA2 || L == LIM_SMOOTHVANALBADA) {
-        const double a2 = hc_fma(a, a, DBL_MIN);
-        double pl = a * bl, pr = a * br;
-        if constexpr (L == LIM_VANALBADA2) {
-            pl = hc_fmax(pl, 0.0);
-            pr = hc_fmax(pr, 0.0);
-        }
-        sl = pl * (a + bl) * hc_rcp(hc_fma(bl, bl, a2));
-        sr = pr * (a + br) * hc_rcp(hc_fma(br, br, a2));
+        double p = a * b;
+        if constexpr (L == LIM_VANALBADA2) p = hc_fmax(p, 0.0);
+        return p * (a + b) * hc_rcp(hc_fma(b, b, hc_fma(a, a, DBL_MIN)));
     } else if constexpr (L == LIM_MINMOD2) {
-        const double lo = hc_fmin(a, 0.0), hi = hc_fmax(a, 0.0);
-        sl = hc_fmin(hc_fmax(bl, lo), hi);
-        sr = hc_fmin(hc_fmax(br, lo), hi);
+        return hc_fmin(hc_fmax(b, hc_fmin(a, 0.0)), hc_fmax(a, 0.0));
     } else {
-        sl = limit_fn<L>(a, bl);
-        sr = limit_fn<L>(a, br);
+        return limit_fn<L>(a, b);
     }
 }
 
 // one branch on the limiter's id per face, straight-line code over the variables
-HC_HD void fused_limit4(int lim, const double* a, const double* bl, const double* br, double* sl, double* sr)
+HC_HD void fused_limit4(int lim, const double* al, const double* bl, const double* ar, const double* br, double* sl, double* sr)
 {
     switch (lim) {
-#define HC_LIM_CASE(L)                                                              \
-    case L:                                                                         \
-        for (int v = 0; v < 4; ++v) fused_limit<L>(a[v], bl[v], br[v], sl[v], sr[v]); \
+#define HC_LIM_CASE(L)                              \
+    case L:                                         \
+        for (int v = 0; v < 4; ++v) {               \
+            sl[v] = fused_limit<L>(al[v], bl[v]);   \
+            sr[v] = fused_limit<L>(ar[v], br[v]);   \
+        }                                           \
         return;
         HC_FOR_EACH_LIMITER(HC_LIM_CASE)
 #undef HC_LIM_CASE
     default:
-        for (int v = 0; v < 4; ++v) fused_limit<LIM_SMOOTHVANALBADA>(a[v], bl[v], br[v], sl[v], sr[v]);
+        for (int v = 0; v < 4; ++v) {
+            sl[v] = fused_limit<LIM_SMOOTHVANALBADA>(al[v], bl[v]);
+            sr[v] = fused_limit<LIM_SMOOTHVANALBADA>(ar[v], br[v]);
+        }
     }
 }
 

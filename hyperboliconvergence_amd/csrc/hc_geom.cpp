@@ -240,15 +240,17 @@ bool uniform_geometry(const GeomInput& in, const GeomOutput& g)
 
 void directional_weights(const std::vector<double>& f, long long nf, std::vector<double>& w)
 {
-    w.resize(4 * nf);
+    w.resize(5 * nf);
     for (long long k = 0; k < nf; ++k) {
         const double n0 = f[FS_N0 * nf + k], n1 = f[FS_N1 * nf + k];
         for (int side = 0; side < 2; ++side) {
             const int s0 = side == 0 ? FS_FL0 : FS_FR0;
             const double x0 = f[s0 * nf + k], x1 = f[(s0 + 1) * nf + k], x2 = f[(s0 + 2) * nf + k];
-            w[2 * side * nf + k] = x0 * n0 + x1 * n1;
-            w[(2 * side + 1) * nf + k] = x1 * n0 + x2 * n1;
+            const double d = f[(side == 0 ? FS_DL : FS_DR) * nf + k];
+            w[2 * side * nf + k] = d * (x0 * n0 + x1 * n1);
+            w[(2 * side + 1) * nf + k] = d * (x1 * n0 + x2 * n1);
         }
+        w[4 * nf + k] = f[FS_DL * nf + k] * f[FS_S1 * nf + k];
     }
 }
 

@@ -42,7 +42,7 @@ bool uniform_geometry(const GeomInput& in, const GeomOutput& g);
 void fp32_slots(const std::vector<double>& f64, long long nf, std::vector<float>& f32);
 
 // the directional weights of the biased LSQ factors in FP64, planes {left 0, left 1, right 0, right 1}:
-// the slots FS_XL0 .. FS_XR1 of a fused context
+// the slots FS_XL0 .. FS_XS of a fused context
 void directional_weights(const std::vector<double>& f64, long long nf, std::vector<double>& w);
 
 }   // namespace hc

@@ -46,8 +46,9 @@ constexpr int FS_CY = FS_DR;
 // factors in place of the factors (two per side)
 constexpr int FS_WL0 = FS_FL0, FS_WL1 = FS_FL1, FS_WR0 = FS_FR0, FS_WR1 = FS_FR1;
 
-// the GPU's FP64 slots of a fused context (hc_fused.hpp) are followed by the same weights in FP64
-enum { FS_XL0 = NSLOT, FS_XL1, FS_XR0, FS_XR1, NSLOT_FUSED };
+// the GPU's FP64 slots of a fused context (hc_fused.hpp) are followed by the same weights in FP64 times the
+// distances to the face, d_L w_L and d_R w_R, and by the left cell's share d_L / (d_L + d_R)
+enum { FS_XL0 = NSLOT, FS_XL1, FS_XR0, FS_XR1, FS_XS, NSLOT_FUSED };
 
 // status bits returned through the C-ABI
 enum StatusBits : unsigned int {
