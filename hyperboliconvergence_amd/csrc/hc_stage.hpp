@@ -309,6 +309,13 @@ struct StageTile {
         }
     }
 
+    // the same for a launch that folds no update, whose loads have no status to report
+    HC_HD static void load(const StageArgs<RF>& a, Smem& s, int i0, int j0, int tid)
+    {
+        unsigned int flag = 0;
+        load(a, s, i0, j0, tid, flag);
+    }
+
     // centre difference of the cells at q-tile positions pl, pr: c_R - c_L, or across a periodic
     // wrap c_R - (c_L - period) (the host geometry's wrap-face operations)
     HC_HD static void centre_diff(const StageArgs<RF>& a, const Smem& s, int pl, int pr, bool wrap, bool isi,
