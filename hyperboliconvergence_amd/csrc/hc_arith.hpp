@@ -19,6 +19,7 @@
 namespace hc {
 
 HC_HD double hc_fma(double a, double b, double c) { return ::fma(a, b, c); }
+HC_HD double hc_copysign(double a, double b) { return ::copysign(a, b); }
 
 // 1 / b: hardware seed (about 2^-24), two Newton steps
 HC_HD double hc_rcp(double b)

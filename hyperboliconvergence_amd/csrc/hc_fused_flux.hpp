@@ -239,8 +239,9 @@ HC_HD void fused_flux(const Species<double>& sp, int vscale, int pscale, double 
 }
 
 // Limiter L of a centred increment a with a biased one b (limiters/limiter.ipp).  van Albada:
-// b a^2 + a b^2 = ab (a + b), and the switch on a b < 0 is a maximum with zero; MinMod: the biased
-// increment clamped to [min(a, 0), max(a, 0)].
+// b a^2 + a b^2 = ab (a + b), and the switch on a b < 0 is a maximum with zero; MinMod: the part of the
+// biased increment that has the sign of a, up to |a| (a NaN increment, beside a NaN state, has none
+// and gives 0 like limit_fn).
 template <int L> HC_HD double fused_limit(double a, double b)
 {
     if constexpr (L == LIM_VANALBADA2 || L == LIM_SMOOTHVANALBADA) {
@@ -248,7 +249,8 @@ template <int L> HC_HD double fused_limit(double a, double b)
         if constexpr (L == LIM_VANALBADA2) p = hc_fmax(p, 0.0);
         return p * (a + b) * hc_rcp(hc_fma(b, b, hc_fma(a, a, DBL_MIN)));
     } else if constexpr (L == LIM_MINMOD2) {
-        return hc_fmin(hc_fmax(b, hc_fmin(a, 0.0)), hc_fmax(a, 0.0));
+        const double sgn = hc_copysign(1.0, a);
+        return hc_copysign(hc_fmin(hc_fmax(b * sgn, 0.0), hc_fabs(a)), a);
     } else {
         return limit_fn<L>(a, b);
     }

@@ -886,12 +886,14 @@ template <class R> HC_HD R limit(int lim, R a, R b)
 template <class R, int N> HC_HD void limit_pairs(int lim, const R* a, const R* bl, const R* br, R* sl, R* sr)
 {
     if constexpr (sizeof(R) == sizeof(double)) {
-        // FP64 MinMod: the biased slope clamped to [min(a, 0), max(a, 0)], 6 operations a variable for 24
+        // FP64 MinMod without a select: the positive part of the biased slope up to max(a, 0) plus its
+        // negative part down to min(a, 0), of which one is zero; a NaN slope (the state beside it is
+        // NaN) has no parts and gives 0, as in limit_fn.  12 operations a variable for 24
         if (lim == LIM_MINMOD2) {
             for (int v = 0; v < N; ++v) {
                 const R lo = hc_fmin(a[v], R(0.)), hi = hc_fmax(a[v], R(0.));
-                sl[v] = hc_fmin(hc_fmax(bl[v], lo), hi);
-                sr[v] = hc_fmin(hc_fmax(br[v], lo), hi);
+                sl[v] = hc_fmin(hc_fmax(bl[v], R(0.)), hi) + hc_fmax(hc_fmin(bl[v], R(0.)), lo);
+                sr[v] = hc_fmin(hc_fmax(br[v], R(0.)), hi) + hc_fmax(hc_fmin(br[v], R(0.)), lo);
             }
             return;
         }
