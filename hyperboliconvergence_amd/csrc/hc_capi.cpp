@@ -405,7 +405,8 @@ bool same_geometry(const GeomOutput& a, const GeomOutput& b)
 // (the part a single-case launch covers, from tile0).
 int build_tiles(hc_context* ctx)
 {
-    const TileShape* shapes = tile_shapes(ctx->precision == HC_PRECISION_MIXED, ctx->cs.law, ctx->cs.flux, ctx->fused);
+    const TileShape* shapes =
+        tile_shapes(ctx->precision == HC_PRECISION_MIXED, ctx->cs.law, ctx->cs.flux, ctx->fused, ctx->wide);
     const int nc = (int)ctx->cases.size();
     for (int k = 0; k < NTILECFG; ++k) {
         long long nt = 0;
@@ -481,8 +482,10 @@ int build_layout(hc_context* ctx)
     long long N = 0, nfi = 0, nfj = 0, br = 0;
     long long gN = 0, gfi = 0, gfj = 0;   // packed geometry: one block per group of equal geometries
     ctx->ngeo = 0;
+    ctx->wide = false;
     for (int ci = 0; ci < nc; ++ci) {
         CaseHost& c = ctx->cases[ci];
+        ctx->wide = ctx->wide || 8 * std::max(c.nfi, c.nfj) >= (1LL << 32) || std::max(c.ni, c.nj) >= (1 << 24) - 1;
         c.cell_off = N;
         c.bref_off = br;
         N += c.N;
@@ -579,11 +582,7 @@ int build_layout(hc_context* ctx)
     HC_HIP(hipMemcpy(ctx->chunks, ch.data(), ch.size() * sizeof(UpdChunk), hipMemcpyHostToDevice));
     ctx->nchunks = (int)ch.size();
     ctx->uni_ok = true;
-    ctx->wide = false;
-    for (const auto& c : ctx->cases) {
-        ctx->uni_ok = ctx->uni_ok && c.uniform;
-        ctx->wide = ctx->wide || 8 * std::max(c.nfi, c.nfj) >= (1LL << 32) || std::max(c.ni, c.nj) >= (1 << 24) - 1;
-    }
+    for (const auto& c : ctx->cases) ctx->uni_ok = ctx->uni_ok && c.uniform;
     ctx->have_case = true;
     return HC_OK;
 }

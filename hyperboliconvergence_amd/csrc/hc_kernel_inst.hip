@@ -34,16 +34,18 @@ template <int K, int UNI, class A> static hipError_t launch_shape(const A& L, hi
 {
     if constexpr (HC_PREC == 64 && hc::fused_euler(HC_LAW, HC_FLUX)) {
         constexpr hc::TileShape S = hc::TILESF[K];
-        // 64-bit offsets only where a plane needs them, and then without the uniform-geometry variant
+        // 64-bit offsets only where a mesh needs them, and then in one shape and without the
+        // uniform-geometry variant (in every shape they were 30 of 150 fused kernels)
+        constexpr hc::TileShape W = hc::TILESW[K];
         if (L.fused && L.wide)
-            return launch<hc::FusedTile<HC_BASIS, HC_FLUX, S.ti, S.tj, S.nt, unsigned long long, 0>, 4>(L, st);
+            return launch<hc::FusedTile<HC_BASIS, HC_FLUX, W.ti, W.tj, W.nt, unsigned long long, 0>, 4>(L, st);
         if (L.fused && L.upd_in)
             return launch<hc::FusedTile<HC_BASIS, HC_FLUX, S.ti, S.tj, S.nt, unsigned, UNI, 1>, 5>(L, st);
         if (L.fused) return launch<hc::FusedTile<HC_BASIS, HC_FLUX, S.ti, S.tj, S.nt, unsigned, UNI>, 5>(L, st);
     }
     // centre staging has nothing to stage on uniform geometry, so a shape that differs from another
     // only by it shares that shape's kernel
-    constexpr hc::TileShape S = hc::tile_shapes(HC_PREC == 32, HC_LAW, HC_FLUX, false)[K];
+    constexpr hc::TileShape S = hc::tile_shapes(HC_PREC == 32, HC_LAW, HC_FLUX, false, false)[K];
     // FP64 in the reference's order takes 91 - 97 VGPRs where the cell phase's inputs are loaded late: five
     // waves per SIMD ask for 96 (AUSM+up in the primitive basis holds them early, at four): the 512x1024
     // gradient 5190 -> 5104 us; the variants that fold an update would spill there and keep four

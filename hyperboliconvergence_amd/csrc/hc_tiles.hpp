@@ -40,9 +40,13 @@ constexpr TileShape TILES32[NTILECFG] = {{8, 32, 256, 0, 0}, {7, 32, 256, 0, 0},
 // halo cells on large ones.  4x32 would give one wave two faces.
 constexpr TileShape TILESF[NTILECFG] = {{7, 16, 256, 1, 1}, {7, 8, 128, 1, 1}, {15, 16, 512, 1, 1}};
 
-constexpr const TileShape* tile_shapes(bool mixed, int law, int flux, bool fused)
+// The same with 64-bit offsets, which only a strip of 2^24 cells along one side takes (a plane of 4 GiB
+// would need more cells than the card holds): one shape, whatever configuration is asked for.
+constexpr TileShape TILESW[NTILECFG] = {TILESF[0], TILESF[0], TILESF[0]};
+
+constexpr const TileShape* tile_shapes(bool mixed, int law, int flux, bool fused, bool wide)
 {
-    if (!mixed && fused) return TILESF;
+    if (!mixed && fused) return wide ? TILESW : TILESF;
     return (!mixed || mixed_wide(law, flux)) ? TILES64 : TILES32;
 }
 
