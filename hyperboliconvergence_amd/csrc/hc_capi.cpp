@@ -163,29 +163,14 @@ __global__ void __launch_bounds__(256) k_soa_to_aos(const double* __restrict__ s
         for (int v = 0; v < nv; ++v) aos[c * nv + v] = soa[v * N + c];
 }
 
-// The slots derived from a direction's FP64 face slots f [NSLOT][nf]: their FP32 copies with the biased LSQ
-// factors replaced by directional weights (fp32_slots' operations), and for a fused context their
-// scaled forms in FP64 as five more planes (directional_weights).  On the host this pass and the upload of the copies
-// were a fifth of setting a case up.
+// The slots derived from a direction's FP64 face slots f [NSLOT][nf]: their FP32 copies, and for a fused
+// context its five further FP64 planes.  On the host this pass and the upload of the copies were a fifth of
+// setting a case up.
 __global__ void __launch_bounds__(256) k_derive_slots(double* __restrict__ f, float* __restrict__ f32, long long nf, int fused)
 {
     for (long long k = (long long)blockIdx.x * 256 + threadIdx.x; k < nf; k += (long long)gridDim.x * 256) {
-        for (int s = 0; s < FS_FL0; ++s) f32[s * nf + k] = (float)f[s * nf + k];
-        const double n0 = f[FS_N0 * nf + k], n1 = f[FS_N1 * nf + k];
-        for (int side = 0; side < 2; ++side) {
-            const int s0 = side == 0 ? FS_FL0 : FS_FR0;
-            const double x0 = f[s0 * nf + k], x1 = f[(s0 + 1) * nf + k], x2 = f[(s0 + 2) * nf + k];
-            const double w0 = x0 * n0 + x1 * n1, w1 = x1 * n0 + x2 * n1;
-            f32[s0 * nf + k] = (float)w0;
-            f32[(s0 + 1) * nf + k] = (float)w1;
-            f32[(s0 + 2) * nf + k] = 0.0f;
-            if (fused) {
-                const double d = f[(side == 0 ? FS_DL : FS_DR) * nf + k];
-                f[(FS_XL0 + 2 * side) * nf + k] = d * w0;
-                f[(FS_XL1 + 2 * side) * nf + k] = d * w1;
-            }
-        }
-        if (fused) f[FS_XS * nf + k] = f[FS_DL * nf + k] * f[FS_S1 * nf + k];
+        fp32_face(f, nf, k, f32);
+        if (fused) scaled_face(f, nf, k, f + FS_XL0 * nf);
     }
 }
 

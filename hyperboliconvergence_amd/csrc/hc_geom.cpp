@@ -241,32 +241,13 @@ bool uniform_geometry(const GeomInput& in, const GeomOutput& g)
 void directional_weights(const std::vector<double>& f, long long nf, std::vector<double>& w)
 {
     w.resize(5 * nf);
-    for (long long k = 0; k < nf; ++k) {
-        const double n0 = f[FS_N0 * nf + k], n1 = f[FS_N1 * nf + k];
-        for (int side = 0; side < 2; ++side) {
-            const int s0 = side == 0 ? FS_FL0 : FS_FR0;
-            const double x0 = f[s0 * nf + k], x1 = f[(s0 + 1) * nf + k], x2 = f[(s0 + 2) * nf + k];
-            const double d = f[(side == 0 ? FS_DL : FS_DR) * nf + k];
-            w[2 * side * nf + k] = d * (x0 * n0 + x1 * n1);
-            w[(2 * side + 1) * nf + k] = d * (x1 * n0 + x2 * n1);
-        }
-        w[4 * nf + k] = f[FS_DL * nf + k] * f[FS_S1 * nf + k];
-    }
+    for (long long k = 0; k < nf; ++k) scaled_face(f.data(), nf, k, w.data());
 }
 
 void fp32_slots(const std::vector<double>& f64, long long nf, std::vector<float>& f32)
 {
-    f32.assign(f64.begin(), f64.end());
-    for (long long k = 0; k < nf; ++k) {
-        const double n0 = f64[FS_N0 * nf + k], n1 = f64[FS_N1 * nf + k];
-        for (int side = 0; side < 2; ++side) {
-            const int s0 = side == 0 ? FS_FL0 : FS_FR0;
-            const double x0 = f64[s0 * nf + k], x1 = f64[(s0 + 1) * nf + k], x2 = f64[(s0 + 2) * nf + k];
-            f32[s0 * nf + k] = float(x0 * n0 + x1 * n1);
-            f32[(s0 + 1) * nf + k] = float(x1 * n0 + x2 * n1);
-            f32[(s0 + 2) * nf + k] = 0.0f;
-        }
-    }
+    f32.resize(NSLOT * nf);
+    for (long long k = 0; k < nf; ++k) fp32_face(f64.data(), nf, k, f32.data());
 }
 
 }   // namespace hc

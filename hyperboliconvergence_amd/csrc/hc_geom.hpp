@@ -36,13 +36,14 @@ int build_geometry(const GeomInput& in, GeomOutput& out);
 // for all faces and cells, with the same bits as the per-face arrays.
 bool uniform_geometry(const GeomInput& in, const GeomOutput& g);
 
+// The slots that contexts derive on the GPU (hc_stage.hpp fp32_face and scaled_face, face by face), here
+// for programs that run the kernels' code on the host.
 // FP32 face slots of the mixed path from the FP64 ones: every slot rounded, except that the two
 // biased LSQ factors become their directional weights w = X'^-1 n (two per side: the slope along
 // n is Q'.w), formed in FP64 and rounded
 void fp32_slots(const std::vector<double>& f64, long long nf, std::vector<float>& f32);
 
-// the directional weights of the biased LSQ factors in FP64, planes {left 0, left 1, right 0, right 1}:
-// the slots FS_XL0 .. FS_XS of a fused context
+// the five planes FS_XL0 .. FS_XS of a fused context: {d_L w_L0, d_L w_L1, d_R w_R0, d_R w_R1, d_L / (d_L + d_R)}
 void directional_weights(const std::vector<double>& f64, long long nf, std::vector<double>& w);
 
 }   // namespace hc

@@ -50,6 +50,42 @@ constexpr int FS_WL0 = FS_FL0, FS_WL1 = FS_FL1, FS_WR0 = FS_FR0, FS_WR1 = FS_FR1
 // distances to the face, d_L w_L and d_R w_R, and by the left cell's share d_L / (d_L + d_R)
 enum { FS_XL0 = NSLOT, FS_XL1, FS_XR0, FS_XR1, FS_XS, NSLOT_FUSED };
 
+// the directional weight w = X'^-1 n of a side (0 left, 1 right) of face k of the slots f
+HC_HD void face_weight(const double* f, long long nf, long long k, int side, double& w0, double& w1)
+{
+    const double* x = f + (side == 0 ? FS_FL0 : FS_FR0) * nf + k;
+    const double n0 = f[FS_N0 * nf + k], n1 = f[FS_N1 * nf + k];
+    w0 = x[0] * n0 + x[nf] * n1;
+    w1 = x[nf] * n0 + x[2 * nf] * n1;
+}
+
+// face k of the FP32 slots: every FP64 slot rounded, with the weights in place of the factors
+HC_HD void fp32_face(const double* f, long long nf, long long k, float* f32)
+{
+    for (int s = 0; s < FS_FL0; ++s) f32[s * nf + k] = (float)f[s * nf + k];
+    for (int side = 0; side < 2; ++side) {
+        float* o = f32 + (side == 0 ? FS_FL0 : FS_FR0) * nf + k;
+        double w0, w1;
+        face_weight(f, nf, k, side, w0, w1);
+        o[0] = (float)w0;
+        o[nf] = (float)w1;
+        o[2 * nf] = 0.0f;
+    }
+}
+
+// face k of the five planes that FS_XL0 .. FS_XS name, at w
+HC_HD void scaled_face(const double* f, long long nf, long long k, double* w)
+{
+    for (int side = 0; side < 2; ++side) {
+        const double d = f[(side == 0 ? FS_DL : FS_DR) * nf + k];
+        double w0, w1;
+        face_weight(f, nf, k, side, w0, w1);
+        w[2 * side * nf + k] = d * w0;
+        w[(2 * side + 1) * nf + k] = d * w1;
+    }
+    w[4 * nf + k] = f[FS_DL * nf + k] * f[FS_S1 * nf + k];
+}
+
 // status bits returned through the C-ABI
 enum StatusBits : unsigned int {
     ST_NONFINITE = 1u,     // non-finite state after an update
