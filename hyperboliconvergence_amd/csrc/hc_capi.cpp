@@ -163,13 +163,13 @@ __global__ void __launch_bounds__(256) k_soa_to_aos(const double* __restrict__ s
         for (int v = 0; v < nv; ++v) aos[c * nv + v] = soa[v * N + c];
 }
 
-// The slots derived from a direction's FP64 face slots f [NSLOT][nf]: their FP32 copies, and for a fused
-// context its five further FP64 planes.  On the host this pass and the upload of the copies were a fifth of
+// The slots derived from a direction's FP64 face slots f [NSLOT][nf]: the FP32 copies (f32, null: none) of a
+// mixed context, and for a fused one its five further FP64 planes.  On the host this pass and the upload of the copies were a fifth of
 // setting a case up.
 __global__ void __launch_bounds__(256) k_derive_slots(double* __restrict__ f, float* __restrict__ f32, long long nf, int fused)
 {
     for (long long k = (long long)blockIdx.x * 256 + threadIdx.x; k < nf; k += (long long)gridDim.x * 256) {
-        fp32_face(f, nf, k, f32);
+        if (f32) fp32_face(f, nf, k, f32);
         if (fused) scaled_face(f, nf, k, f + FS_XL0 * nf);
     }
 }
@@ -353,14 +353,14 @@ template <class RF> void fill_rec(const hc_context* ctx, const CaseHost& c, Case
     r.m.ccx = ctx->ccx + c.geo_cell_off;
     r.m.ccy = ctx->ccy + c.geo_cell_off;
     if constexpr (sizeof(RF) == 8) {
-        r.m.fi = ctx->fi + ctx->nslot64() * c.geo_fi_off;
-        r.m.fj = ctx->fj + ctx->nslot64() * c.geo_fj_off;
+        r.m.fi = ctx->fi + ctx->nslot_i * c.geo_fi_off;
+        r.m.fj = ctx->fj + ctx->nslot_j * c.geo_fj_off;
     } else {
-        r.m.fi = ctx->fi32 + NSLOT * c.geo_fi_off;
-        r.m.fj = ctx->fj32 + NSLOT * c.geo_fj_off;
+        r.m.fi = ctx->fi32 ? ctx->fi32 + NSLOT * c.geo_fi_off : nullptr;
+        r.m.fj = ctx->fj32 ? ctx->fj32 + NSLOT * c.geo_fj_off : nullptr;
     }
-    r.m.fi64 = ctx->fi + ctx->nslot64() * c.geo_fi_off;
-    r.m.fj64 = ctx->fj + ctx->nslot64() * c.geo_fj_off;
+    r.m.fi64 = ctx->fi + ctx->nslot_i * c.geo_fi_off;
+    r.m.fj64 = ctx->fj + ctx->nslot_j * c.geo_fj_off;
     for (int d = 0; d < 2; ++d) {
         r.m.period_i[d] = c.cs.period_i[d];
         r.m.period_j[d] = c.cs.period_j[d];
@@ -443,10 +443,79 @@ int build_tiles(hc_context* ctx)
     return HC_OK;
 }
 
-void derive_slots(hc_context* ctx, double* f, float* f32, long long nf)
+// planes of FP64 face slots that the kernels of the context's precision read
+int planes(const hc_context* ctx)
 {
-    const unsigned grid = (unsigned)std::min<long long>((nf + 255) / 256, 8192);
-    hipLaunchKernelGGL(k_derive_slots, dim3(grid), dim3(256), 0, ctx->stream, f, f32, nf, ctx->fused ? 1 : 0);
+    return ctx->fused && ctx->precision == HC_PRECISION_FP64 ? NSLOT_FUSED : NSLOT;
+}
+
+// The slots that the context's precision reads beside the uploaded ones, formed on the GPU.  Each precision
+// holds its own only (112 B a cell for the FP32 copies, 80 for a fused context's planes): of the device
+// memory of a cell, 600 to 800 B, the largest mesh that fits is bound by it.
+int derive_slots(hc_context* ctx)
+{
+    const bool mixed = ctx->precision == HC_PRECISION_MIXED, fused = planes(ctx) == NSLOT_FUSED;
+    if (mixed && !ctx->fi32) HC_HIP(hipMalloc(&ctx->fi32, NSLOT * ctx->gfi_tot * sizeof(float)));
+    if (mixed && !ctx->fj32) HC_HIP(hipMalloc(&ctx->fj32, NSLOT * ctx->gfj_tot * sizeof(float)));
+    auto derive = [&](double* f, float* f32, long long nf) {
+        const unsigned grid = (unsigned)std::min<long long>((nf + 255) / 256, 8192);
+        hipLaunchKernelGGL(k_derive_slots, dim3(grid), dim3(256), 0, ctx->stream, f, f32, nf, fused ? 1 : 0);
+    };
+    for (int ci = 0; ci < (int)ctx->cases.size(); ++ci) {
+        const CaseHost& c = ctx->cases[ci];
+        if (c.geo != ci || !(mixed || fused)) continue;
+        derive(ctx->fi + ctx->nslot_i * c.geo_fi_off, mixed ? ctx->fi32 + NSLOT * c.geo_fi_off : nullptr, c.nfi);
+        derive(ctx->fj + ctx->nslot_j * c.geo_fj_off, mixed ? ctx->fj32 + NSLOT * c.geo_fj_off : nullptr, c.nfj);
+    }
+    HC_HIP(hipGetLastError());
+    HC_HIP(hipStreamSynchronize(ctx->stream));
+    return HC_OK;
+}
+
+// Moves the FP64 slots of one direction into as many planes as the context's precision reads
+int resize_planes(hc_context* ctx, bool dir_i)
+{
+    double*& f = dir_i ? ctx->fi : ctx->fj;
+    int& have = dir_i ? ctx->nslot_i : ctx->nslot_j;
+    const int want = planes(ctx);
+    if (have == want) return HC_OK;
+    double* n = nullptr;
+    const hipError_t e = hipMalloc(&n, want * (dir_i ? ctx->gfi_tot : ctx->gfj_tot) * sizeof(double));
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return want < have ? HC_OK : hipfail(ctx, e, "face slots");   // too many planes do as well
+    }
+    for (int ci = 0; ci < (int)ctx->cases.size(); ++ci) {
+        const CaseHost& c = ctx->cases[ci];
+        if (c.geo != ci) continue;
+        const long long off = dir_i ? c.geo_fi_off : c.geo_fj_off, nf = dir_i ? c.nfi : c.nfj;
+        const hipError_t ec =
+            hipMemcpyAsync(n + want * off, f + have * off, NSLOT * nf * sizeof(double), hipMemcpyDeviceToDevice, ctx->stream);
+        if (ec != hipSuccess) {
+            (void)hipStreamSynchronize(ctx->stream);
+            (void)hipFree(n);
+            return hipfail(ctx, ec, "face slots");
+        }
+    }
+    HC_HIP(hipStreamSynchronize(ctx->stream));
+    free_dev(f);
+    f = n;
+    have = want;
+    return HC_OK;
+}
+
+// The slots of the other precision, which ctx->precision has just become, in place of those held.  The
+// FP32 copies go first, so that a mixed context has the room to become an FP64 one.
+int switch_slots(hc_context* ctx)
+{
+    if (ctx->precision == HC_PRECISION_FP64) {
+        free_dev(ctx->fi32);
+        free_dev(ctx->fj32);
+    }
+    int r = resize_planes(ctx, true);
+    if (r == HC_OK) r = resize_planes(ctx, false);
+    if (r == HC_OK) r = derive_slots(ctx);
+    return r;
 }
 
 // device layout of all cases: packed arrays, case records, tile tables, update chunks
@@ -508,11 +577,11 @@ int build_layout(hc_context* ctx)
     HC_HIP(hipMalloc(&ctx->cvol, gN * sizeof(double)));
     HC_HIP(hipMalloc(&ctx->ccx, gN * sizeof(double)));
     HC_HIP(hipMalloc(&ctx->ccy, gN * sizeof(double)));
-    const long long nslot = ctx->nslot64();
+    ctx->gfi_tot = gfi;
+    ctx->gfj_tot = gfj;
+    const long long nslot = ctx->nslot_i = ctx->nslot_j = planes(ctx);
     HC_HIP(hipMalloc(&ctx->fi, nslot * gfi * sizeof(double)));
     HC_HIP(hipMalloc(&ctx->fj, nslot * gfj * sizeof(double)));
-    HC_HIP(hipMalloc(&ctx->fi32, NSLOT * gfi * sizeof(float)));
-    HC_HIP(hipMalloc(&ctx->fj32, NSLOT * gfj * sizeof(float)));
     for (int ci = 0; ci < nc; ++ci) {
         CaseHost& c = ctx->cases[ci];
         if (c.geo == ci) {
@@ -523,15 +592,12 @@ int build_layout(hc_context* ctx)
             double* fj = ctx->fj + nslot * c.geo_fj_off;
             HC_HIP(hipMemcpy(fi, c.g.fi.data(), c.g.fi.size() * sizeof(double), hipMemcpyHostToDevice));
             HC_HIP(hipMemcpy(fj, c.g.fj.data(), c.g.fj.size() * sizeof(double), hipMemcpyHostToDevice));
-            derive_slots(ctx, fi, ctx->fi32 + NSLOT * c.geo_fi_off, c.nfi);
-            derive_slots(ctx, fj, ctx->fj32 + NSLOT * c.geo_fj_off, c.nfj);
-            HC_HIP(hipGetLastError());
         }
         const GeomInput gin{c.ni, c.nj, nullptr, {c.cs.bc[0], c.cs.bc[1], c.cs.bc[2], c.cs.bc[3]}, {0.0, 0.0}, {0.0, 0.0}};
         c.uniform = uniform_geometry(gin, c.g);
         c.X = std::move(c.g.X);
     }
-    HC_HIP(hipStreamSynchronize(ctx->stream));   // the derived slots are written
+    if (const int r = derive_slots(ctx)) return r;
     for (auto& c : ctx->cases) c.g = GeomOutput{};   // the device holds it now
     // state, accumulators, per-case slots
     for (auto& b : ctx->q) {
@@ -1150,11 +1216,19 @@ int hc_set_precision(hc_context* ctx, int precision)
     if (ctx->building) return fail(ctx, HC_ERR_STATE, "batch not finished (hc_batch_end)");
     ctx->precision = precision;
     if (!ctx->have_case) return HC_OK;
-    // the tile tables depend on the precision's tile shapes: rebuild them, keeping the cases' data
+    // the derived slots and the tile tables are the precision's: form them anew, keeping the cases' data
     HC_HIP(hipSetDevice(ctx->device));
     HC_HIP(hipStreamSynchronize(ctx->stream));
     drop_graph(ctx);
-    const int r = build_tiles(ctx);
+    int r = switch_slots(ctx);
+    if (r) {   // no room for them: back to the slots that the context had
+        const std::string err = ctx->err;
+        ctx->precision = precision == HC_PRECISION_MIXED ? HC_PRECISION_FP64 : HC_PRECISION_MIXED;
+        if (switch_slots(ctx) != HC_OK || build_tiles(ctx) != HC_OK) ctx->have_case = false;
+        ctx->err = err;
+        return r;
+    }
+    r = build_tiles(ctx);
     if (r) return r;
     ctx->tuned = false;
     ctx->tile_cfg = ctx->tile_mode >= 0 ? ctx->tile_mode : 0;

@@ -60,6 +60,7 @@ struct hc_context {
     std::vector<RkPlan> plans;
     int nslots = 0;
     long long Ntot = 0, nfi_tot = 0, nfj_tot = 0, brows_tot = 0;
+    long long gfi_tot = 0, gfj_tot = 0;   // faces of the geometry blocks held on the device
     // device buffers
     double *cvol = nullptr, *ccx = nullptr, *ccy = nullptr, *fi = nullptr, *fj = nullptr;
     float *fi32 = nullptr, *fj32 = nullptr;
@@ -82,7 +83,7 @@ struct hc_context {
     int tile_mode = -1;
     int tile_cfg = 0;
     bool fused = false;            // FP64 runs the fused Euler tile (hc_fused.hpp)
-    long long nslot64() const { return fused ? hc::NSLOT_FUSED : hc::NSLOT; }   // planes of the FP64 face slots
+    int nslot_i = 0, nslot_j = 0;  // planes of the FP64 face slots fi, fj: NSLOT_FUSED where a fused tile reads them
     bool wide = false;             // some case's planes pass 32-bit byte offsets (LaunchArgs::wide)
     bool uni_ok = false;           // every case has uniform geometry
     bool uni_enable = true;        // use the uniform-geometry kernels when uni_ok (hc_set_uniform_geometry)
