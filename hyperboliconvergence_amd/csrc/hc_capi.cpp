@@ -518,6 +518,22 @@ int switch_slots(hc_context* ctx)
     return r;
 }
 
+// The second deferred-residual buffer of chained steps, in contexts that chain: one-stage tables with a
+// global step in FP64, whose update has the same bits in either kernel (the mixed objects contract it by its
+// surroundings, and a state must not depend on how the steps were split over calls), within 32-bit offsets.
+// It is allocated last, and steps stay single where it does not fit.
+void chain_buffer(hc_context* ctx)
+{
+    const bool want = ctx->cs.nstages == 1 && ctx->cs.dt_mode == HC_DT_GLOBAL && ctx->precision == HC_PRECISION_FP64 &&
+                      !ctx->wide;
+    if (!want) {
+        free_dev(ctx->tmp2);
+    } else if (!ctx->tmp2 && hipMalloc(&ctx->tmp2, (size_t)ctx->nv * ctx->Ntot * sizeof(double)) != hipSuccess) {
+        (void)hipGetLastError();
+        ctx->tmp2 = nullptr;
+    }
+}
+
 // device layout of all cases: packed arrays, case records, tile tables, update chunks
 int build_layout(hc_context* ctx)
 {
@@ -607,7 +623,6 @@ int build_layout(hc_context* ctx)
     ctx->cur = 0;
     if (ctx->nslots > 0) HC_HIP(hipMalloc(&ctx->acc, (size_t)ctx->nslots * nv * N * sizeof(double)));
     HC_HIP(hipMalloc(&ctx->tmp, (size_t)nv * N * sizeof(double)));
-    if (ctx->cs.nstages == 1 && ctx->cs.dt_mode == HC_DT_GLOBAL) HC_HIP(hipMalloc(&ctx->tmp2, (size_t)nv * N * sizeof(double)));
     HC_HIP(hipMalloc(&ctx->lam0, N * sizeof(double)));
     HC_HIP(hipMalloc(&ctx->res, (size_t)(nv + 1) * N * sizeof(double)));
     HC_HIP(hipMalloc(&ctx->bref, (size_t)br * nv * sizeof(double)));
@@ -634,6 +649,7 @@ int build_layout(hc_context* ctx)
     ctx->nchunks = (int)ch.size();
     ctx->uni_ok = true;
     for (const auto& c : ctx->cases) ctx->uni_ok = ctx->uni_ok && c.uniform;
+    chain_buffer(ctx);
     ctx->have_case = true;
     return HC_OK;
 }
@@ -822,14 +838,9 @@ int enqueue_step(hc_context* ctx)
     return HC_OK;
 }
 
-// Whether consecutive steps are chained (enqueue_steps): one-stage tables with a global step in FP64, whose
-// update has the same bits in either kernel (the mixed objects contract it by its surroundings, and a
-// state must not depend on how the steps were split over calls).  Event pairs around each kernel keep the
-// kernels of single steps, and so do planes beyond 32-bit offsets
-bool chains(const hc_context* ctx)
-{
-    return ctx->tmp2 && ctx->precision == HC_PRECISION_FP64 && !ctx->wide && ctx->profiling != 1;
-}
+// Whether consecutive steps are chained (enqueue_steps): contexts that hold the buffer for it
+// (chain_buffer).  Event pairs around each kernel keep the kernels of single steps
+bool chains(const hc_context* ctx) { return ctx->tmp2 && ctx->profiling != 1; }
 
 // n steps.  One-stage tables with a global step run n + 2 kernels instead of 3 n: the residual kernel of
 // step k + 1 forms the update of step k while it loads its tiles (and stores it, the step's result), so
@@ -1230,6 +1241,7 @@ int hc_set_precision(hc_context* ctx, int precision)
     }
     r = build_tiles(ctx);
     if (r) return r;
+    chain_buffer(ctx);
     ctx->tuned = false;
     ctx->tile_cfg = ctx->tile_mode >= 0 ? ctx->tile_mode : 0;
     return HC_OK;

@@ -83,3 +83,22 @@ def test_switched_precision_gives_the_bits_of_a_new_context(first, then):
             ctx.set_tiles(0)
             out.append((ctx.residual(), ctx.step(5), ctx.get_state()))
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][2], out[1][2])
+
+
+def test_second_residual_buffer_of_chained_steps():
+    """One-stage tables with a global step: FP64 contexts hold a second deferred residual, mixed ones do not."""
+    import hyperboliconvergence_amd as hca
+    from test_gpu_chained import _table
+    N, rest = NI * NJ, REST - 8 * 4   # no accumulator
+    cfg = _table(_cfg(hca.FLUX_ROE_FACEFRAME, NI, NJ, True), "ssp11")
+    FP64, MIXED = hca.PRECISION_FP64, hca.PRECISION_MIXED
+    with _context(_cfg(hca.FLUX_ROE, 8, 16), FP64):
+        pass
+    for first, then, extra in ((FP64, FP64, WEIGHTS + 8 * 4), (MIXED, MIXED, FP32), (FP64, MIXED, FP32),
+                               (MIXED, FP64, WEIGHTS + 8 * 4)):
+        before = _free()
+        with _context(cfg, first) as ctx:
+            if then != first:
+                ctx.set_precision(then)
+            used = (before - _free()) / N
+        assert 0 <= used - (SLOTS + extra + rest) <= 30, (first, then, used, SLOTS + extra + rest)
