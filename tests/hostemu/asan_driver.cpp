@@ -3,7 +3,8 @@
 // store of the kernels' index arithmetic checked against the buffers it addresses).
 //
 // Input (native byte order): int32[8] {ni, nj, precision, nsteps, tile configuration (+16: the
-// uniform-geometry kernels where the case allows them), adjoint, nv, sizeof(hc_case_desc)}, the hc_case_desc bytes, then doubles: nodes [ni+1][nj+1][2],
+// uniform-geometry kernels where the case allows them, +32 or +64: the fused Euler tile with 32- or 64-bit
+// offsets, +128: folded and chained updates), adjoint, nv, sizeof(hc_case_desc)}, the hc_case_desc bytes, then doubles: nodes [ni+1][nj+1][2],
 // q [ni][nj][nv], bref [2nj+2ni][nv] and, when adjoint != 0, qd [ni][nj][nv] and ybar [ni][nj][nv].
 // Output, doubles: residual [ni][nj][nv+1], the state after nsteps [ni][nj][nv], the time and the
 // status; when adjoint != 0 also the tangent residual [ni][nj][nv+1] and its derivative
@@ -17,6 +18,8 @@
 extern "C" {
 int emu_set_tile_config(int cfg);
 int emu_set_uniform_geometry(int enable);
+int emu_set_fused(int mode);
+int emu_set_fold(int on);
 int emu_residual(const hc_case_desc* cs, int ni, int nj, const double* nodes, const double* q, const double* bref,
                  int precision, double* res, unsigned int* status);
 int emu_integrate(const hc_case_desc* cs, int ni, int nj, const double* nodes, double* q, const double* bref,
@@ -66,7 +69,9 @@ int main(int argc, char** argv)
         return 2;
     }
     if (emu_set_tile_config(tiles & 15) != 0) return 3;
-    emu_set_uniform_geometry(tiles >> 4);
+    emu_set_uniform_geometry((tiles >> 4) & 1);
+    if (emu_set_fused((tiles >> 5) & 3) != 0) return 3;
+    emu_set_fold((tiles >> 7) & 1);
 
     std::vector<double> res(N * (nv + 1)), qs(q), tail(2);
     unsigned int st = 0;
