@@ -39,9 +39,13 @@ template <int K, int UNI, class A> static hipError_t launch_shape(const A& L, hi
         constexpr hc::TileShape W = hc::TILESW[K];
         if (L.fused && L.wide)
             return launch<hc::FusedTile<HC_BASIS, HC_FLUX, W.ti, W.tj, W.nt, unsigned long long, 0>, 4>(L, st);
+        // Five waves per SIMD where they can be had.  15x16 holds 58 KB of LDS, two groups a CU: four.  The
+        // folded general tile would spill 20 registers for the fifth, which gains nothing (1000x901 AUSM+up
+        // 1265 us for 6 steps at four waves, 1261 - 1271 at five; 144x96 one-stage 408 for 50, 410 at five)
+        constexpr int W64 = S.nt > 256 ? 4 : 5, WF64 = UNI ? W64 : 4;
         if (L.fused && L.upd_in)
-            return launch<hc::FusedTile<HC_BASIS, HC_FLUX, S.ti, S.tj, S.nt, unsigned, UNI, 1>, 5>(L, st);
-        if (L.fused) return launch<hc::FusedTile<HC_BASIS, HC_FLUX, S.ti, S.tj, S.nt, unsigned, UNI>, 5>(L, st);
+            return launch<hc::FusedTile<HC_BASIS, HC_FLUX, S.ti, S.tj, S.nt, unsigned, UNI, 1>, WF64>(L, st);
+        if (L.fused) return launch<hc::FusedTile<HC_BASIS, HC_FLUX, S.ti, S.tj, S.nt, unsigned, UNI>, W64>(L, st);
     }
     // centre staging has nothing to stage on uniform geometry, so a shape that differs from another
     // only by it shares that shape's kernel
