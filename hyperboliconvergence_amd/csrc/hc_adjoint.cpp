@@ -270,7 +270,7 @@ int minf_total(hc_context* ctx)
     return HC_OK;
 }
 
-// stage s of the fused kernel from q_in into q_out (not in place), plans and accumulators as in a step
+// stage s of the stage kernel from q_in into q_out (not in place), plans and accumulators as in a step
 int stage_into(hc_context* ctx, int s, const double* q_in, const double* q0, double* q_out)
 {
     LaunchArgs<double> L = launch_args<double>(ctx);
@@ -541,7 +541,7 @@ int hc_tangent_steps(hc_context* ctx, int nsteps, const double* qdot0, const dou
             hipLaunchKernelGGL(k_rk_tangent, dim3(blocks(len)), dim3(256), 0, ctx->stream, s.qdot[st + 1], s.qdot[0],
                                tk, ctx->cs.beta[st] * dt, ctx->cvol, N, nv);
             HC_HIP(hipGetLastError());
-            // state: stage outputs through the fused kernel, the last one in place
+            // state: stage outputs through the stage kernel, the last one in place
             double* out = st == ns - 1 ? s.qtmp : s.stage[st + 1];
             if ((r = stage_into(ctx, st, in, qn, out))) return r;
             in = out;

@@ -69,8 +69,10 @@ HC_HD double hc_root(double x, double& inv)
 #endif
 }
 
-// a / b and sqrt(x) with the bits of the correctly rounded operations: the compiler's own sequences
-// without the scaling of extreme exponents (9 instructions instead of 11, and 13 instead of 18).  The
+// a / b and sqrt(x) with the bits of the correctly rounded operations: Newton-Raphson on the reciprocal with
+// Markstein's final quotient correction, and Goldschmidt's coupled iteration with two residual corrections of
+// the root, without the scaling of extreme exponents that library sequences begin and end with (9
+// instructions instead of 11, and 13 instead of 18).  The
 // fixup keeps zeros, infinities and NaNs as they are; bits agree for operands and quotients of
 // magnitude 2^-900 .. 2^900 and roots of 2^-767 and more.  The mixed-precision objects keep the
 // compiler's sequences (their few FP64 divisions gain nothing: the 48-case batch ran 4 % slower with these).

@@ -13,9 +13,10 @@
 //               96 cylinders 13.87 -> 13.59 ms for 10)
 //   4. cells  : R = F_left - F_right of the four faces (the wall flux of the far sides is stored
 //               negated), then the Runge-Kutta accumulation and the update as StageTile has them
-// Sums at the sides are in another order than the oracle's and products are fused: results agree to
-// rounding (1e-13 of the residual), and are the same bits in every tile shape, since every fused
-// operation is explicit.
+// Sums at the sides are in another order than the oracle's and products are fused: residuals agree to
+// rounding of the face fluxes they are differences of, 2e-15 of the largest (vortex boxes of 64^2 to 400^2
+// cells, every flux; relative to the residual itself that grows with the mesh, 3e-14 to 3e-13 there), and
+// are the same bits in every tile shape, since every fused operation is explicit.
 //
 // Bound: latency of the load phase, then instruction issue (96 cylinders, a wavefront's 15.1k cycles: waits
 // for the record and the tile 5.4k, metric 1.7k, faces 3.8k, cells 1.8k, barriers 2.4k; VALU busy 61 % at
@@ -424,9 +425,7 @@ template <int BASIS, int FLUX, int TI, int TJ, int NTHR, class Off, int UNI, int
         double fac;
         if (a.dt_mode == 0) {
             fac = hc_div(p.beta * (folded(a) ? a.dt_in : a.dtslot[0]), ci.vol);
-        } else if (a.dt_mode == 2) {
-            fac = hc_div(p.beta * a.cfl, ci.vol);   // fixed step: cfl holds dt
-        } else {
+        } else {   // local steps (fixed ones keep the ordered tile)
             const double l0 = a.stage == 0 ? lam : ci.lam0;
             if (a.stage == 0) put(a.lam0, o, lam);
             fac = hc_div(p.beta * a.cfl, l0);

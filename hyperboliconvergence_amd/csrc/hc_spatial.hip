@@ -2,9 +2,9 @@
 // context: Q metric, ghost-value update, spectral radius and the forward-Euler updates.  They
 // serve callers that run the time loop themselves on host arrays (the C++ drop-in's xmetrics /
 // qmetrics / boundaryUpdate / spectralRadius / eulerForwardUpdateGlobal / Local); hc_step runs
-// the same arithmetic fused into the stage kernel.  Host arrays are staged through the context's
+// the same scheme fused into the stage kernel.  Host arrays are staged through the context's
 // device buffers between steps (those buffers hold no step state then).  Compiled with
-// -ffp-contract=off: each result is bit-identical to the fused kernel's and to the oracle's.
+// -ffp-contract=off: each result is bit-identical to the oracle's, and to StageTile's in FP64.
 #include "hc_context.hpp"
 
 #include <hip/hip_runtime.h>
