@@ -5,14 +5,13 @@
 // buffer rotation and Runge-Kutta plans as the C-ABI.  Tests use it to check the
 // kernels' arithmetic and LDS indexing against the oracle without a GPU.  It is
 // never part of the product library.
-#include "hc_fused.hpp"
+#include "hosttiles.hpp"
+
 #include "hc_geom.hpp"
-#include "hc_stage.hpp"
 #include "hc_tiles.hpp"
 #include "hcamd.h"
 
 #include <cfloat>
-#include <memory>
 #include <vector>
 
 using namespace hc;
@@ -86,41 +85,6 @@ int g_uniform = 0;
 // stage-0 update folded into stage 1's loads
 int g_fold = 0;
 
-template <class T, class RF> void run_tiles(const StageArgs<RF>& a)
-{
-    constexpr int TI = T::TILE_I, TJ = T::TILE_J;
-    const int tiles_i = (a.m.ni + TI - 1) / TI, tiles_j = (a.m.nj + TJ - 1) / TJ;
-    const int ntiles = tiles_i * tiles_j;
-    auto sp = std::make_unique<typename T::Smem>();
-    typename T::Smem& s = *sp;
-    std::vector<unsigned int> flag(T::NT);
-    for (int b = 0; b < ntiles; ++b) {
-        const int t = xcd_tile(b, ntiles);
-        const int i0 = (t / tiles_j) * TI, j0 = (t % tiles_j) * TJ;
-        for (auto& f : flag) f = 0;
-        std::vector<typename T::Geo> g0(T::NT);
-        for (int tid = 0; tid < T::NT; ++tid) {
-            T::load(a, s, i0, j0, tid, flag[tid]);
-            T::prefetch(a, i0, j0, tid, g0[tid]);
-        }
-        for (int tid = 0; tid < T::NT; ++tid) T::qmetric(a, s, i0, j0, tid);
-        for (int tid = 0; tid < T::NT; ++tid) T::faces(a, s, i0, j0, tid, flag[tid], g0[tid]);
-        std::vector<double> red(T::NT);
-        std::vector<typename T::CellIn> ci(T::NT);
-        for (int tid = 0; tid < T::NT; ++tid) T::prefetch_cell(a, i0, j0, tid, ci[tid]);
-        for (int tid = 0; tid < T::NT; ++tid) T::cells(a, s, i0, j0, tid, flag[tid], red[tid], ci[tid]);
-        double m = 0.0;
-        unsigned int f = 0;
-        for (int tid = 0; tid < T::NT; ++tid) {
-            m = fmax(m, red[tid]);
-            f |= flag[tid];
-        }
-        if (a.mode == MODE_GLOBAL_STAGE0 && dbl_bits(m) > *a.maxslot) *a.maxslot = dbl_bits(m);
-        *a.status |= f;
-    }
-    if (a.reset_max) *a.maxslot = dbl_bits(DBL_MIN);
-}
-
 template <int LAW, int BASIS, int FLUX, class RF, int TI, int TJ, int NT, int CST, int GPF, int UNI>
 void run_stage_t(const StageArgs<RF>& a)
 {
@@ -132,30 +96,14 @@ bool g_case_uniform = false;
 // the fused Euler tile (hc_fused.hpp) in FP64: 1 with 32-bit offsets, 2 with 64-bit ones
 int g_fused = 0;
 
-template <int BASIS, int FLUX, int K> void run_fused_flux(const StageArgs<double>& a)
-{
-    constexpr TileShape S = TILESF[K];
-    if (g_uniform && g_case_uniform) run_tiles<FusedTile<BASIS, FLUX, S.ti, S.tj, S.nt, unsigned, 1>>(a);
-    else if (g_fused == 2 && K == 0) run_tiles<FusedTile<BASIS, FLUX, TILESF[0].ti, TILESF[0].tj, TILESF[0].nt, unsigned long long, 0>>(a);
-    else run_tiles<FusedTile<BASIS, FLUX, S.ti, S.tj, S.nt, unsigned, 0>>(a);
-}
-
-template <int BASIS, int K> void run_fused(int flux, const StageArgs<double>& a)
-{
-    switch (flux) {
-    case 0: run_fused_flux<BASIS, 0, K>(a); break;
-    case 1: run_fused_flux<BASIS, 1, K>(a); break;
-    case 4: run_fused_flux<BASIS, 4, K>(a); break;
-    case 5: run_fused_flux<BASIS, 5, K>(a); break;
-    default: run_fused_flux<BASIS, 6, K>(a); break;
-    }
-}
-
-template <int LAW, int BASIS, int FLUX, class RF, int TI, int TJ, int NT, int CST, int GPF>
+// WIDE: the shapes are those of the mixed kernels that keep FP64 face states (all FP64 kernels take them)
+template <int LAW, int BASIS, int FLUX, class RF, bool WIDE, int TI, int TJ, int NT, int CST, int GPF>
 void run_stage(const StageArgs<RF>& a)
 {
-    if (g_uniform && g_case_uniform) run_stage_t<LAW, BASIS, FLUX, RF, TI, TJ, NT, 0, GPF, 1>(a);
-    else run_stage_t<LAW, BASIS, FLUX, RF, TI, TJ, NT, CST, GPF, 0>(a);
+    if constexpr (sizeof(RF) == 8 || mixed_wide(LAW, FLUX) == WIDE) {
+        if (g_uniform && g_case_uniform) run_stage_t<LAW, BASIS, FLUX, RF, TI, TJ, NT, 0, GPF, 1>(a);
+        else run_stage_t<LAW, BASIS, FLUX, RF, TI, TJ, NT, CST, GPF, 0>(a);
+    }
 }
 
 template <int LAW, int BASIS, class RF> void run_update(const StageArgs<RF>& a)
@@ -167,26 +115,26 @@ template <int LAW, int BASIS, class RF> void run_update(const StageArgs<RF>& a)
     *a.status |= flag;
 }
 
-template <class RF, int TI, int TJ, int NT, int CST, int GPF> void dispatch_stage(const hc_case_desc& cs, const StageArgs<RF>& a)
+template <class RF, bool WIDE, int TI, int TJ, int NT, int CST, int GPF> void dispatch_stage(const hc_case_desc& cs, const StageArgs<RF>& a)
 {
     const int key = cs.law * 100 + cs.basis * 10 + cs.flux;
     switch (key) {
-    case 0: run_stage<0, 0, 0, RF, TI, TJ, NT, CST, GPF>(a); break;
-    case 1: run_stage<0, 0, 1, RF, TI, TJ, NT, CST, GPF>(a); break;
-    case 100: run_stage<1, 0, 0, RF, TI, TJ, NT, CST, GPF>(a); break;
-    case 101: run_stage<1, 0, 1, RF, TI, TJ, NT, CST, GPF>(a); break;
-    case 102: run_stage<1, 0, 2, RF, TI, TJ, NT, CST, GPF>(a); break;
-    case 103: run_stage<1, 0, 3, RF, TI, TJ, NT, CST, GPF>(a); break;
-    case 104: run_stage<1, 0, 4, RF, TI, TJ, NT, CST, GPF>(a); break;
-    case 105: run_stage<1, 0, 5, RF, TI, TJ, NT, CST, GPF>(a); break;
-    case 106: run_stage<1, 0, 6, RF, TI, TJ, NT, CST, GPF>(a); break;
-    case 110: run_stage<1, 1, 0, RF, TI, TJ, NT, CST, GPF>(a); break;
-    case 111: run_stage<1, 1, 1, RF, TI, TJ, NT, CST, GPF>(a); break;
-    case 112: run_stage<1, 1, 2, RF, TI, TJ, NT, CST, GPF>(a); break;
-    case 113: run_stage<1, 1, 3, RF, TI, TJ, NT, CST, GPF>(a); break;
-    case 114: run_stage<1, 1, 4, RF, TI, TJ, NT, CST, GPF>(a); break;
-    case 115: run_stage<1, 1, 5, RF, TI, TJ, NT, CST, GPF>(a); break;
-    case 116: run_stage<1, 1, 6, RF, TI, TJ, NT, CST, GPF>(a); break;
+    case 0: run_stage<0, 0, 0, RF, WIDE, TI, TJ, NT, CST, GPF>(a); break;
+    case 1: run_stage<0, 0, 1, RF, WIDE, TI, TJ, NT, CST, GPF>(a); break;
+    case 100: run_stage<1, 0, 0, RF, WIDE, TI, TJ, NT, CST, GPF>(a); break;
+    case 101: run_stage<1, 0, 1, RF, WIDE, TI, TJ, NT, CST, GPF>(a); break;
+    case 102: run_stage<1, 0, 2, RF, WIDE, TI, TJ, NT, CST, GPF>(a); break;
+    case 103: run_stage<1, 0, 3, RF, WIDE, TI, TJ, NT, CST, GPF>(a); break;
+    case 104: run_stage<1, 0, 4, RF, WIDE, TI, TJ, NT, CST, GPF>(a); break;
+    case 105: run_stage<1, 0, 5, RF, WIDE, TI, TJ, NT, CST, GPF>(a); break;
+    case 106: run_stage<1, 0, 6, RF, WIDE, TI, TJ, NT, CST, GPF>(a); break;
+    case 110: run_stage<1, 1, 0, RF, WIDE, TI, TJ, NT, CST, GPF>(a); break;
+    case 111: run_stage<1, 1, 1, RF, WIDE, TI, TJ, NT, CST, GPF>(a); break;
+    case 112: run_stage<1, 1, 2, RF, WIDE, TI, TJ, NT, CST, GPF>(a); break;
+    case 113: run_stage<1, 1, 3, RF, WIDE, TI, TJ, NT, CST, GPF>(a); break;
+    case 114: run_stage<1, 1, 4, RF, WIDE, TI, TJ, NT, CST, GPF>(a); break;
+    case 115: run_stage<1, 1, 5, RF, WIDE, TI, TJ, NT, CST, GPF>(a); break;
+    case 116: run_stage<1, 1, 6, RF, WIDE, TI, TJ, NT, CST, GPF>(a); break;
     default: break;
     }
 }
@@ -206,12 +154,12 @@ template <int K> void stage_shape(Emu& e, StageArgs<double>& a64, StageArgs<floa
 {
     constexpr TileShape S64 = TILES64[K], S32 = TILES32[K];
     if (g_fused && e.precision != HC_PRECISION_MIXED && e.cs.law == HC_LAW_EULER) {
-        if (e.cs.basis == HC_BASIS_CONSERVED) run_fused<0, K>(e.cs.flux, a64);
-        else run_fused<1, K>(e.cs.flux, a64);
-    } else if (e.precision != HC_PRECISION_MIXED) dispatch_stage<double, S64.ti, S64.tj, S64.nt, S64.cst, S64.gpf>(e.cs, a64);
+        const bool uniform = g_uniform && g_case_uniform;
+        run_fused(e.cs.basis, e.cs.flux, K, g_fused == 2 && !uniform, uniform, a64);
+    } else if (e.precision != HC_PRECISION_MIXED) dispatch_stage<double, true, S64.ti, S64.tj, S64.nt, S64.cst, S64.gpf>(e.cs, a64);
     else if (mixed_wide(e.cs.law, e.cs.flux))
-        dispatch_stage<float, S64.ti, S64.tj, S64.nt, S64.cst, S64.gpf>(e.cs, a32);
-    else dispatch_stage<float, S32.ti, S32.tj, S32.nt, S32.cst, S32.gpf>(e.cs, a32);
+        dispatch_stage<float, true, S64.ti, S64.tj, S64.nt, S64.cst, S64.gpf>(e.cs, a32);
+    else dispatch_stage<float, false, S32.ti, S32.tj, S32.nt, S32.cst, S32.gpf>(e.cs, a32);
 }
 
 void stage(Emu& e, StageArgs<double>& a64, StageArgs<float>& a32)
