@@ -164,8 +164,8 @@ __global__ void __launch_bounds__(256) k_soa_to_aos(const double* __restrict__ s
 }
 
 // The slots derived from a direction's FP64 face slots f [NSLOT][nf]: the FP32 copies (f32, null: none) of a
-// mixed context, and for a fused one its five further FP64 planes.  On the host this pass and the upload of the copies were a fifth of
-// setting a case up.
+// mixed context, and for a fused one its five further FP64 planes.  On the host this pass and the upload of
+// the copies were a fifth of setting a case up.
 __global__ void __launch_bounds__(256) k_derive_slots(double* __restrict__ f, float* __restrict__ f32, long long nf, int fused)
 {
     for (long long k = (long long)blockIdx.x * 256 + threadIdx.x; k < nf; k += (long long)gridDim.x * 256) {
@@ -226,6 +226,7 @@ int fail(hc_context* c, int code, const std::string& msg)
 
 int hipfail(hc_context* c, hipError_t e, const char* where)
 {
+    (void)hipGetLastError();   // reported here; the check after the next launch would find it again
     return fail(c, HC_ERR_HIP, std::string(where) + ": " + hipGetErrorString(e));
 }
 
@@ -450,8 +451,8 @@ int planes(const hc_context* ctx)
 }
 
 // The slots that the context's precision reads beside the uploaded ones, formed on the GPU.  Each precision
-// holds its own only (112 B a cell for the FP32 copies, 80 for a fused context's planes): of the device
-// memory of a cell, 600 to 800 B, the largest mesh that fits is bound by it.
+// holds its own only: 112 B a cell for the FP32 copies, 80 for a fused context's planes, of some 550 B in
+// all, which bound the largest mesh that fits.
 int derive_slots(hc_context* ctx)
 {
     const bool mixed = ctx->precision == HC_PRECISION_MIXED, fused = planes(ctx) == NSLOT_FUSED;

@@ -105,7 +105,11 @@ int hc_set_mesh(hc_context* ctx, int ni, int nj, const double* nodes);
  */
 int hc_set_case(hc_context* ctx, const hc_case_desc* desc);
 
-/* FP64 throughout (default) or FP32 face arithmetic with FP64 state, RK and metrics. */
+/*
+ * FP64 throughout (default) or FP32 face arithmetic with FP64 state, RK and metrics.  On a built case the
+ * device copies that the other precision reads are exchanged for this one's; without the device memory for
+ * them the call returns HC_ERR_HIP and the context stays as it was.
+ */
 int hc_set_precision(hc_context* ctx, int precision);
 
 /* Boundary reference values, SolutionField::boundary[b](k,1) (solutionField/solutionField.h:56-91). */
