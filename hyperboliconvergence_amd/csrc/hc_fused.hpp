@@ -21,7 +21,7 @@
 // Bound: latency of the load phase, then instruction issue (96 cylinders, a wavefront's 15.1k cycles: waits
 // for the record and the tile 5.4k, metric 1.7k, faces 3.8k, cells 1.8k, barriers 2.4k; VALU busy 61 % at
 // 4.2 waves a SIMD).  Against StageTile: the same 96 cylinders 18.9 -> 13.6 ms for 10 steps, a 2048x2048
-// AUSM+up box 7.66 -> 2.99 ms for 4, a 256x512 cylinder 1.44 -> 1.00 ms for 20.
+// AUSM+up box 7.66 -> 2.99 ms for 4, a 256x512 cylinder 1.44 -> 0.97 ms for 20.
 // Tried and slower: six waves with the fluxes stored over the state tile (spills off uniform geometry: 96
 // cylinders 13.98 -> 15.07 ms), a persistent loop that loads the next tile during the cell phase (2048x2048
 // 3.15 -> 3.76 ms).
